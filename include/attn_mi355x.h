@@ -350,7 +350,10 @@ int attn_decode_plan(size_t kv_len, size_t num_heads, size_t num_kv_heads, size_
                      size_t kv_stride, const void* q, const void* k_cache,
                      const void* v_cache, uint32_t out[5]);
 
-/* Prefill path chosen for a shape: 0 generic, 1 MFMA. */
+/* Prefill path chosen for a shape: 1 = the MFMA tiles of four query heads per KV
+ * head and head_dim 128, 0 = any other layout (head_dim 64 and 128 with 16-byte
+ * aligned rows run the 64-rows-per-wave MFMA kernel from 64 tokens, everything
+ * else the generic kernel). */
 int attn_prefill_plan(const void* q, const void* k, const void* v, const void* out,
                       size_t num_heads, size_t num_kv_heads, size_t head_dim, size_t q_stride,
                       size_t kv_stride);
@@ -374,7 +377,8 @@ int attn_prefill_plan(const void* q, const void* k, const void* v, const void* o
  * workgroup per head and 32-query tile, its keys split over the waves and
  * combined through LDS, as 8 waves of 32 keys up to 32 tokens, 4 waves of
  * 64-key tiles up to 256 and 4 waves each streaming every 4th 32-key unit
- * above; 1 = never, also no key halves; 2 = 4 waves of 64-key tiles (up to
+ * above (query tiles of 64 tokens instead of 32 from 11/16 of a workgroup per
+ * CU to two, 705 tokens for 16 heads); 1 = never, also no key halves; 2 = 4 waves of 64-key tiles (up to
  * 256 tokens); 3 = 8 waves of 32 keys (up to 256 tokens); 4 = the
  * streaming form at any length), "prefill_key_halves" (0 = automatic: from
  * 1025 to 4096 tokens, unless "prefill_waves" or "prefill_split_keys" is

@@ -574,6 +574,11 @@ int attn_prefill(const attn_f16_t* q, const attn_f16_t* k, const attn_f16_t* v,
     a.q_tiles = (uint32_t)((seq_len + 63) / 64);
     a.scale_log2 = scale_log2_for(head_dim);
     const int path = plan_prefill(a);
+    int device = 0;
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return (int)e;
+    if (const int parts = rows64_parts(a, path == 1, device))
+        return (int)launch_prefill_rows64(a, parts, path == 1, stream);
     if (path == 1) return (int)launch_prefill_kernel(a, path, stream);
     GenericAttnArgs g{};
     g.q = a.q;

@@ -1,5 +1,6 @@
 // Generic grouped-query attention for shapes the MFMA paths do not cover
-// (head_dim != 128, unaligned or odd strides, e.g. the reference's Flash-Decode
+// (prefill: head_dim other than 64 and 128, fewer than 64 tokens of the layouts
+// prefill_rows64.hip takes; decode: head_dim != 128; unaligned or odd strides, e.g. the reference's Flash-Decode
 // known-answer test with D = 32 and kv_stride = kv_dim + 17).
 //
 // One 256-thread workgroup per (query row, query head).  Keys are streamed in

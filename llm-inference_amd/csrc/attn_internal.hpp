@@ -259,6 +259,10 @@ struct PrefillArgs {
 
 int plan_prefill(const PrefillArgs& a);  // 0 generic, 1 MFMA
 hipError_t launch_prefill_kernel(const PrefillArgs& a, int path, hipStream_t stream);
+// the 64-rows-per-wave kernel (prefill_rows64.hip): key parts per head (2 or 4)
+// for a shape, 0 when another kernel takes it; mfma: plan_prefill is 1
+int rows64_parts(const PrefillArgs& a, bool mfma, int device);
+hipError_t launch_prefill_rows64(const PrefillArgs& a, int parts, bool mfma, hipStream_t stream);
 
 // generic attention (one workgroup per query row and head); also the decode
 // fallback for head_dim != 128 or unaligned strides

@@ -1,0 +1,119 @@
+"""The 64-rows-per-wave prefill kernel (prefill_rows64.hip): the layouts that
+attention_generic took before (64-dim heads, KV heads shared by other than a
+multiple of four query heads), against that kernel on the same inputs, and the
+middle range of the model's layout, against the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import assert_close
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(N, Hq, Hkv, D, pad, seed, grow=False):
+    """Q rows of a fused [Q | K | V] buffer, K and V rows of a cache; `pad`
+    elements past each row.  grow: scores rise along the keys, so that the
+    running maximum is raised again and again."""
+    rng = np.random.default_rng(seed)
+    qs, ks = (Hq + 2 * Hkv) * D + pad, Hkv * D + pad
+    q = rng.standard_normal((N, qs)).astype(np.float16)
+    k = rng.standard_normal((N, ks)).astype(np.float16)
+    v = rng.standard_normal((N, ks)).astype(np.float16)
+    if grow:
+        k = (k * np.linspace(0.1, 6.0, N)[:, None]).astype(np.float16)
+    return q, k, v, qs, ks
+
+
+def run(attn, device, q, k, v, Hq, Hkv, D, qs, ks):
+    N = q.shape[0]
+    d = [torch.from_numpy(x.copy()).to(device) for x in (q, k, v)]
+    guard = 64
+    out = torch.full((N * Hq * D + 2 * guard,), 77.0, dtype=torch.float16, device=device)
+    attn.prefill(*d, out[guard:].data_ptr(), N, Hq, Hkv, D, qs, ks)
+    torch.cuda.synchronize()
+    o = out.cpu().numpy()
+    assert (o[:guard] == 77).all() and (o[-guard:] == 77).all(), "write outside out"
+    return o[guard:-guard].reshape(N, Hq * D)
+
+
+def run_generic(attn, device, *args):
+    attn.set_option("prefill_force_generic", 1)
+    try:
+        return run(attn, device, *args)
+    finally:
+        attn.set_option("prefill_force_generic", 0)
+
+
+def assert_as_generic(got, ref, v):
+    # both sum fp32 products of fp32 (or 22-bit) weights: they differ by fp32
+    # rounding of sums of terms up to max|v| (2e-6 of it, ~30 roundings of
+    # 2^-24), and then by at most one rounding to fp16 (2^-10 of the value)
+    ref, got = ref.astype(np.float64), got.astype(np.float64)
+    bound = 2.0 ** -10 * np.abs(ref) + 2e-6 * np.abs(v.astype(np.float64)).max() + 2.0 ** -24
+    bad = ~(np.abs(got - ref) <= bound)
+    assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4], np.abs(got - ref).max())
+
+
+# one and several key units per wave, the last query tile full, one row and one
+# block long; past two rounds of workgroups (1041 and 576 of them) two key parts
+@pytest.mark.parametrize("Hq,Hkv,D,N,pad", [
+    (16, 16, 128, 64, 0), (16, 16, 128, 65, 0), (16, 8, 128, 97, 8), (6, 2, 128, 130, 24),
+    (5, 5, 128, 300, 0), (16, 16, 128, 1000, 0), (32, 16, 128, 1100, 8),
+    (16, 4, 64, 64, 0), (16, 4, 64, 95, 8), (8, 8, 64, 128, 0), (3, 1, 64, 129, 16),
+    (16, 4, 64, 1025, 0), (16, 8, 64, 4161, 0)])
+@pytest.mark.parametrize("grow", [False, True])
+def test_rows64_as_generic(attn, gpu, Hq, Hkv, D, N, pad, grow):
+    print(f"[case] rows64 Hq={Hq} Hkv={Hkv} D={D} N={N} pad={pad} grow={grow}", flush=True)
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, pad, N + Hq, grow)
+    args = (q, k, v, Hq, Hkv, D, qs, ks)
+    got = run(attn, gpu, *args)
+    assert_as_generic(got, run_generic(attn, gpu, *args), v)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,N", [(16, 16, 128, 300), (16, 4, 64, 300), (16, 8, 64, 4200)])
+def test_rows64_infinities_and_nans(attn, gpu, Hq, Hkv, D, N):
+    """An infinity or NaN in K or V reaches exactly the rows that see its key."""
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, 0, 5)
+    v[N - 60, 3] = np.inf
+    v[N - 40, D + 7] = np.nan
+    k[N - 20, 1] = np.nan
+    v[N - 10, 5] = -np.inf
+    print(f"[case] rows64 inf/nan Hq={Hq} Hkv={Hkv} D={D} N={N}", flush=True)
+    args = (q, k, v, Hq, Hkv, D, qs, ks)
+    got, ref = run(attn, gpu, *args), run_generic(attn, gpu, *args)
+    assert np.isfinite(ref[:N - 60]).all() and not np.isfinite(ref[N - 1]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    assert_as_generic(np.where(fine, got, 0), np.where(fine, ref, 0),
+                      np.where(np.isfinite(v), v, 0))
+
+
+# 16 heads: the first and the last length of the range (192 and 256 workgroups),
+# with one row and 32 rows in the last tile; 32, 24 and 12 heads (up to 512)
+@pytest.mark.parametrize("Hq,Hkv,N,pad", [
+    (16, 4, 704, 0), (16, 4, 705, 0), (16, 4, 736, 8), (16, 4, 800, 0), (16, 4, 1024, 0),
+    (32, 8, 353, 0), (32, 4, 1023, 8), (24, 3, 700, 0), (12, 3, 1000, 0)])
+@pytest.mark.parametrize("grow", [False, True])
+def test_rows64_model_layout(attn, gpu, Hq, Hkv, N, pad, grow):
+    D = 128
+    print(f"[case] rows64 model layout Hq={Hq} Hkv={Hkv} N={N} grow={grow}", flush=True)
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, pad, 3 * N, grow)
+    got = run(attn, gpu, q, k, v, Hq, Hkv, D, qs, ks)
+    rows = np.unique(np.concatenate([np.arange(0, N, 17), np.arange(max(0, N - 66), N)]))
+    _, e32 = oracle.attention(q.view(np.uint16).ravel(), k.view(np.uint16).ravel(),
+                              v.view(np.uint16).ravel(), N, Hq, Hkv, D, qs, ks, N, causal=True,
+                              rows=rows)
+    assert_close(got[rows].reshape(-1).view(np.uint16), e32.reshape(-1), 2e-3, 1e-2, f"N={N}")
+
+
+def test_rows64_prefix_invariance(attn, gpu):
+    """A row depends on the rows up to it only, bit for bit, also where the
+    prefix ends inside its query tile."""
+    q, k, v, qs, ks = inputs(1020, 16, 4, 128, 0, 8)
+    whole = run(attn, gpu, q, k, v, 16, 4, 128, qs, ks)
+    for n in (705, 766, 960):
+        part = run(attn, gpu, q[:n], k[:n], v[:n], 16, 4, 128, qs, ks)
+        assert np.array_equal(part.view(np.uint16), whole[:n].view(np.uint16)), n
