@@ -663,6 +663,36 @@ int attn_decode(const attn_f16_t* q, const attn_f16_t* k_cache, const attn_f16_t
     const DecodePlan p = plan_decode((uint32_t)kv_len, (uint32_t)num_heads,
                                      (uint32_t)num_kv_heads, (uint32_t)head_dim, kvs, q,
                                      k_cache, v_cache, device, true);
+    // 64-dim heads: the split and merge kernels of decode_d64.hip where the call
+    // brings a workspace and asks for no node (a caller of the one generic node
+    // below may patch that node alone)
+    if (p.path == 0 && head_dim == 64 && !attention_node && !merge_node &&
+        get_option(kOptDecodeForceGeneric) == 0) {
+        DecodeD64Args d{};
+        d.q = reinterpret_cast<const f16*>(q);
+        d.k = reinterpret_cast<const f16*>(k_cache);
+        d.v = reinterpret_cast<const f16*>(v_cache);
+        d.out = reinterpret_cast<f16*>(out);
+        d.part_out = partial_out;
+        d.part_max = partial_max;
+        d.part_sum = partial_sum;
+        d.kv_stride = kvs;
+        d.kv_len = (uint32_t)kv_len;
+        d.num_heads = (uint32_t)num_heads;
+        d.num_kv_heads = (uint32_t)num_kv_heads;
+        d.group = (uint32_t)(num_heads / num_kv_heads);
+        d.capacity = (uint32_t)((kv_len + ATTN_KV_CHUNK - 1) / ATTN_KV_CHUNK);
+        d.scale_log2 = scale_log2_for(head_dim);
+        if (plan_decode_d64(d, device)) {
+            e = launch_decode_d64_split(d, stream);
+            if (e != hipSuccess) return (int)e;
+            remember_launch<DecodeD64Args>(stream);
+            e = launch_decode_d64_merge(d, stream);
+            if (e != hipSuccess) return (int)e;
+            remember_launch<DecodeD64Args>(stream);
+            return 0;
+        }
+    }
     if (p.path == 0) {
         // one kernel: both node handles name it (the merge patcher is a no-op)
         GenericAttnArgs g{};
@@ -938,6 +968,51 @@ int attn_update_rope_decode_nodes(hipGraphExec_t graph_exec, hipGraphNode_t atte
     return 0;
 }
 
+// Either node of a captured 64-dim decode moves both to kv_len: a caller that
+// looked up one node after the call knows the pair as one decode.  The other
+// is the merge's dependency or the split's dependent of the same call (same
+// output).
+static int patch_decode_d64(hipGraphExec_t graph_exec, hipGraphNode_t node, const NodeView& view,
+                            size_t kv_len) {
+    int device = 0;
+    hipError_t e = node_device(view, &device);
+    if (e != hipSuccess) return (int)e;
+    DecodeD64Args a = *reinterpret_cast<const DecodeD64Args*>(view.arg);
+    a.kv_len = (uint32_t)kv_len;
+    if (!plan_decode_d64(a, device)) return (int)hipErrorInvalidValue;
+    const bool is_merge = view.params.func == decode_d64_merge_symbol();
+    hipGraphNode_t near[16];
+    size_t n = sizeof(near) / sizeof(near[0]);
+    e = is_merge ? hipGraphNodeGetDependencies(node, near, &n)
+                 : hipGraphNodeGetDependentNodes(node, near, &n);
+    if (e != hipSuccess) return (int)e;
+    n = n < sizeof(near) / sizeof(near[0]) ? n : sizeof(near) / sizeof(near[0]);
+    hipGraphNode_t other = nullptr;
+    NodeView other_view;
+    for (size_t i = 0; i < n && !other; ++i) {
+        hipGraphNodeType type;
+        if (hipGraphNodeGetType(near[i], &type) != hipSuccess || type != hipGraphNodeTypeKernel)
+            continue;
+        if (view_node(near[i], other_view) != hipSuccess) continue;
+        if (is_merge ? !is_decode_d64_split(other_view.params.func)
+                     : other_view.params.func != decode_d64_merge_symbol())
+            continue;
+        if (reinterpret_cast<const DecodeD64Args*>(other_view.arg)->out == a.out) other = near[i];
+    }
+    if (!other) return (int)hipErrorInvalidValue;
+    void* args[1] = {&a};
+    for (int m = 0; m < 2; ++m) {
+        const bool this_one = (m == 1) == is_merge;
+        hipKernelNodeParams params = this_one ? view.params : other_view.params;
+        params.kernelParams = args;
+        params.extra = nullptr;
+        if (m == 0) params.gridDim = decode_d64_grid(a);
+        e = hipGraphExecKernelNodeSetParams(graph_exec, this_one ? node : other, &params);
+        if (e != hipSuccess) return (int)e;
+    }
+    return 0;
+}
+
 static int patch_decode_node(hipGraphExec_t graph_exec, hipGraphNode_t node, size_t kv_len,
                              bool merge) {
     if (kv_len == 0 || !fits_u32(kv_len)) return (int)hipErrorInvalidValue;
@@ -955,6 +1030,8 @@ static int patch_decode_node(hipGraphExec_t graph_exec, hipGraphNode_t node, siz
         params.extra = nullptr;
         return (int)hipGraphExecKernelNodeSetParams(graph_exec, node, &params);
     }
+    if (is_decode_d64_split(params.func) || params.func == decode_d64_merge_symbol())
+        return patch_decode_d64(graph_exec, node, view, kv_len);
     int device = 0;
     if (params.func == merge_out_proj_symbol(false)) {
         // the merge fused into o_proj: its decode arguments follow kv_len

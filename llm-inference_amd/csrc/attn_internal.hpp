@@ -239,6 +239,35 @@ bool out_proj_fused_ok(const OutProjArgs& a);
 hipError_t launch_merge_out_proj(const OutProjArgs& a, hipStream_t stream, bool rope);
 const void* merge_out_proj_symbol(bool rope);
 
+// Split decode of 64-dim heads (decode_d64.hip): fp32 partial states of nsplit
+// chunks per query head, then their merge.
+struct DecodeD64Args {
+    const f16* q;        // [Hq][64] packed
+    const f16* k;        // cache rows, kv_stride elements apart
+    const f16* v;
+    f16* out;            // [Hq][64] packed
+    float* part_out;     // [Hq][nsplit][64]  (workspace)
+    float* part_max;     // [Hq][nsplit]      (workspace, log2 domain)
+    float* part_sum;     // [Hq][nsplit]
+    uint64_t kv_stride;
+    uint32_t kv_len;     // patched per decode step
+    uint32_t num_heads;
+    uint32_t num_kv_heads;
+    uint32_t group;
+    uint32_t nsplit;     // patched
+    uint32_t chunk;      // patched
+    uint32_t capacity;   // states per head of the call's workspace: what its kv_len asks for
+    float scale_log2;
+};
+// fills nsplit and chunk; false: attention_generic takes the call
+bool plan_decode_d64(DecodeD64Args& a, int device);
+const void* decode_d64_split_symbol(const DecodeD64Args& a);
+const void* decode_d64_merge_symbol();
+bool is_decode_d64_split(const void* fn);
+dim3 decode_d64_grid(const DecodeD64Args& a);
+hipError_t launch_decode_d64_split(const DecodeD64Args& a, hipStream_t stream);
+hipError_t launch_decode_d64_merge(const DecodeD64Args& a, hipStream_t stream);
+
 // ------------------------------------------------------------- prefill
 struct PrefillArgs {
     const f16* q;       // [N] rows, q_stride elements apart, Hq heads of D

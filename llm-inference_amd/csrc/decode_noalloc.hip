@@ -81,7 +81,8 @@ extern "C" int attn_decode_noalloc(const attn_f16_t* q, const attn_f16_t* k_cach
                                      k_cache, v_cache, device, true);
     if (p.path == 0) {
         // shapes off the MFMA path take attn_decode's generic kernel, which
-        // has no partial states
+        // has no partial states (64-dim heads too: their split kernels need a
+        // workspace, and calls of these shapes may overlap)
         return attn_decode(q, k_cache, v_cache, out, nullptr, nullptr, nullptr, 1, kv_len,
                            kv_len - 1, num_heads, num_kv_heads, head_dim, 0, kv_stride, stream,
                            nullptr, nullptr);
