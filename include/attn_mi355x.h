@@ -82,7 +82,11 @@ int attn_prefill(const attn_f16_t* q, const attn_f16_t* k, const attn_f16_t* v,
  * (one workgroup per KV head writes the output; with merge_node the merge
  * kernel follows and exits at once, so that an updater can move the pair to
  * a longer context); other shapes enqueue one generic kernel and both
- * handles receive it.
+ * handles receive it, except head_dim 64 without node handles (16-byte
+ * aligned tensors, a workspace): a split and a merge kernel of their own, in
+ * fp32 like the generic kernel, which attn_update_decode_node and
+ * attn_update_merge_node patch together through either node (never past the
+ * states that the capturing call's kv_len asks for).
  * Replaces launch_causal_attention_decode (kernels.hpp:104-123) and
  * launch_causal_attention_decode_vectorized (kernels.hpp:127-146;
  * causal_attention.hip.cpp:840-972). */
@@ -152,7 +156,8 @@ int attn_update_rope_decode_nodes(hipGraphExec_t graph_exec, hipGraphNode_t atte
  * q_stride unused) without a caller workspace, for callers that cannot
  * allocate device memory (code under graph capture that must not call
  * hipMalloc, tight serving loops, harnesses that forbid it).  Same plan,
- * kernels and output bits as attn_decode; the partial states go to a
+ * kernels and output bits as attn_decode (head_dim 64: the generic kernel, equal within
+ * fp32 rounding); the partial states go to a
  * library-owned array of ATTN_DECODE_NOALLOC_SCRATCH_BYTES per GPU (held
  * until the process ends; its address is looked up once per device on the
  * first call there).  A plan whose states exceed the array (more than

@@ -17,7 +17,9 @@
 //  * Everything past the fp16 inputs is fp32, as in attention_generic: vector
 //    ALU products (the matrix cores would take fp16 weights), fp32 states in the
 //    caller's workspace.  The arithmetic (4 query heads: ~130 instructions per
-//    wave and 8 keys) is a tenth of the time even at 4 heads per KV head.
+//    wave and 8 keys) is a small part of the time.
+// Measured (one MI355X): a decode token over 12 layers at 3000 keys, 16/4
+// heads, projections included, 2849 -> 215 us.
 #include "attn_internal.hpp"
 
 #include <algorithm>
