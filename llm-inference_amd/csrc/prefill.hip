@@ -408,13 +408,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void prefill_d128(PrefillArgs a) {
                 if constexpr (kShift) pb[r] = (f16)fast_exp2(x);
                 else pb[r] = (f16)fast_exp2(__builtin_fmaf(x, a.scale_log2, mneg));
             }
-            // row sum of the fp16 weights the PV product uses, two per
-            // v_dot2_f32_f16 (fp32 accumulate)
+            // row sum of the fp16 weights the PV product uses, in fp32
 #pragma unroll
-            for (int r = 0; r < 8; r += 2) {
-                const f16x2 pair = {pb[r], pb[r + 1]};
-                psum = __builtin_amdgcn_fdot2(pair, f16x2{(f16)1.0f, (f16)1.0f}, psum, false);
-            }
+            for (int r = 0; r < 8; r += 2)
+                psum = add_pair(psum, f16x2{pb[r], pb[r + 1]});
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) o[dt] = mfma32(va[dt], pb, o[dt]);
         }
@@ -789,10 +786,8 @@ __global__ __launch_bounds__(64 * kSkWaves, 1) void prefill_sk32(PrefillArgs a) 
             for (int r = 0; r < 8; ++r)
                 pb[r] = (f16)fast_exp2(__builtin_fmaf(s[8 * ks + r], a.scale_log2, mneg));
 #pragma unroll
-            for (int r = 0; r < 8; r += 2) {
-                const f16x2 pair = {pb[r], pb[r + 1]};
-                psum = __builtin_amdgcn_fdot2(pair, f16x2{(f16)1.0f, (f16)1.0f}, psum, false);
-            }
+            for (int r = 0; r < 8; r += 2)
+                psum = add_pair(psum, f16x2{pb[r], pb[r + 1]});
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) o[dt] = mfma32(va[dt], pb, o[dt]);
         }
@@ -995,10 +990,8 @@ __global__ __launch_bounds__(64 * kSknWaves, 1) void prefill_skn(PrefillArgs a) 
             for (int r = 0; r < 8; ++r)
                 pb[r] = (f16)fast_exp2(__builtin_fmaf(s[8 * ks + r], a.scale_log2, mneg));
 #pragma unroll
-            for (int r = 0; r < 8; r += 2) {
-                const f16x2 pair = {pb[r], pb[r + 1]};
-                psum = __builtin_amdgcn_fdot2(pair, f16x2{(f16)1.0f, (f16)1.0f}, psum, false);
-            }
+            for (int r = 0; r < 8; r += 2)
+                psum = add_pair(psum, f16x2{pb[r], pb[r + 1]});
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) o[dt] = mfma32(va[dt], pb, o[dt]);
         }

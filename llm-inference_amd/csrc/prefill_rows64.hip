@@ -155,16 +155,6 @@ __device__ __forceinline__ void copy16(u32x4 r, uint32_t lds, uint32_t voff) {
         : "memory", "scc");
 }
 
-// sum + both values of a pair (v_fma_mix_f32: v_dot2_f32_f16 takes the MFMAs'
-// pipe, 18 cycles per instruction next to them)
-__device__ __forceinline__ float add_pair(float sum, f16x2 w) {
-    asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "+v"(sum)
-        : "v"(w));
-    return sum;
-}
-
 // weight pairs w[0..7] (and w[8..15]) as the B operands of their PV steps
 template <bool LO>
 __device__ __forceinline__ void operands(f16x8 (&p)[4], const f16x2 (&w)[16]) {
