@@ -26,6 +26,7 @@
 //  * Workgroups are dispatched round-robin over the 8 XCDs; the tile grid is
 //    split over them (2 x 4 when it divides: each XCD owns half the token
 //    tiles and a quarter of the feature tiles, whose W rows stay in its L2).
+//  * Up to 256 tokens (K >= 1024) the kernels of qkv_short.hip replace it.
 //  * From 7168 tokens (N a multiple of 384, Y 16-byte aligned) a 256 x 384
 //    tile of 8 waves (qkv_gemm_wide, below) replaces it: a third of the X
 //    re-reads and 1.5x the MFMA work per staged byte; identical results.
@@ -593,6 +594,10 @@ hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t 
         return hipGetLastError();
     }
     if (use_wide(a)) return launch_wide(a, fused, stream);
+    int device = 0;
+    if (hipError_t e = hipGetDevice(&device)) return e;
+    if (const int tile = qkv_short_tile(a, device); tile >= 0)
+        return launch_qkv_gemm_short(a, tile, fused, stream);
     switch (qkv_gemm_wmt(a.M)) {
         case 1: return launch_mfma<1>(a, fused, stream);
         case 2: return launch_mfma<2>(a, fused, stream);
