@@ -73,7 +73,6 @@ struct QkvGemmArgs {
 };
 
 bool qkv_gemm_mfma_ok(const QkvGemmArgs& a);
-int qkv_gemm_wmt(uint32_t M);
 // fused: only when qkv_gemm_mfma_ok (hipErrorInvalidValue otherwise)
 hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t stream);
 // qkv_short.hip: the tile for a short prompt, or -1 (qkv_gemm_mfma_ok is the

@@ -27,9 +27,9 @@
 //    split over them (2 x 4 when it divides: each XCD owns half the token
 //    tiles and a quarter of the feature tiles, whose W rows stay in its L2).
 //  * Up to 256 tokens (K >= 1024) the kernels of qkv_short.hip replace it.
-//  * From 7168 tokens (N a multiple of 384, Y 16-byte aligned) a 256 x 384
-//    tile of 8 waves (qkv_gemm_wide, below) replaces it: a third of the X
-//    re-reads and 1.5x the MFMA work per staged byte; identical results.
+//  * For long prompts (N a multiple of 384 or 256, Y 16-byte aligned) a tile of
+//    256 x 384 or 256 x 256 with 8 waves (qkv_gemm_wide, below) replaces it:
+//    fewer X re-reads and more MFMA work per staged byte; identical results.
 //  * Epilogue: fp32 -> fp16 (the GEMM's output rounding), then for the fused
 //    kernel the rope.hip.cpp:44-58 rotation on those fp16 values (fp32
 //    products each rounded, no contraction): Q rows written rotated, K rows
@@ -42,9 +42,6 @@ namespace attn {
 namespace {
 
 constexpr int kBK = 64;      // k-values per stage
-// automatic use of the wide tile: from 28 token tiles (224 of the 256 CUs
-// busy at N = 3072); below that the 256 x 128 tile keeps more CUs busy
-constexpr uint32_t kWideMinTokens = 7168;
 constexpr int kRowH = kBK;   // halves per LDS row (128 B, no padding)
 constexpr int kThreads = 256;
 
@@ -90,18 +87,17 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     constexpr int kADma = BM * 8 / 64;        // 1 KiB DMA instructions per X stage
     constexpr int kBDma = 128 * 8 / 64;       // ... per W stage (16)
     constexpr int kDmaPerWave = (kADma + kBDma) / 4;
-    // vmcnt value that leaves one stage of this wave's DMA outstanding
-    constexpr int kWaitOne = 0x0F70 | (kDmaPerWave & 15) | ((kDmaPerWave >> 4) << 14);
-    static_assert(kDmaPerWave < 64, "vmcnt range");
+    constexpr int kStages = 3;
+    constexpr uint32_t kStageA = BM * kRowH * 2, kStage = kStageA + 128 * kRowH * 2;  // bytes
+    // vmcnt value that leaves kStages - 2 stages of this wave's DMA outstanding
+    constexpr int kLeft = (kStages - 2) * kDmaPerWave;
+    constexpr int kWaitOne = 0x0F70 | (kLeft & 15) | ((kLeft >> 4) << 14);
+    static_assert(kLeft < 64, "vmcnt range");
+    static_assert(kStages * kStage <= 160 * 1024, "LDS");
 
-    // three stages; the DMA is issued by dma16 (inline assembly), so the only
-    // waits between stages are the explicit vmcnt + barrier of each step
-    __shared__ __attribute__((aligned(16))) f16 sa0[BM * kRowH];
-    __shared__ __attribute__((aligned(16))) f16 sa1[BM * kRowH];
-    __shared__ __attribute__((aligned(16))) f16 sa2[BM * kRowH];
-    __shared__ __attribute__((aligned(16))) f16 sb0[128 * kRowH];
-    __shared__ __attribute__((aligned(16))) f16 sb1[128 * kRowH];
-    __shared__ __attribute__((aligned(16))) f16 sb2[128 * kRowH];
+    // the DMA is issued by dma16 (inline assembly), so the only waits between
+    // stages are the explicit vmcnt + barrier of each step
+    __shared__ __attribute__((aligned(16))) f16 lds[kStages * kStage / 2];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -136,23 +132,27 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
         const uint32_t row = p >> 3, slot = p & 7u;
         voff[t] = row * row_bytes + 16u * (slot ^ ((row >> 1) & 7u));
     }
-    auto stage = [&](uint32_t kt, f16* sa, f16* sb) {
+    const uint32_t KT = K / kBK;
+    const uint32_t lds0 = lds_addr(lds) + 1024u * (uint32_t)wave;
+    u32x4 rx, rw;
+    uint32_t la;
+    auto target = [&](uint32_t kt, uint32_t buf) __attribute__((always_inline)) {
         // resources start at k-value 64 kt of the tile's first row and end at
-        // the last row of the matrix: rows past M / N read as zero
+        // the last row of the matrix: rows past M / N read as zero, and so do
+        // whole stages past K (they keep the wait of every step the same)
         const uint32_t k0b = kt * (uint32_t)kBK * 2u;
-        const u32x4 rx = rsrc_words(reinterpret_cast<const char*>(xb) + k0b,
-                                    rows_x * row_bytes - k0b);
-        const u32x4 rw = rsrc_words(reinterpret_cast<const char*>(wb) + k0b,
-                                    rows_w * row_bytes - k0b);
-        const uint32_t la = lds_addr(sa) + 1024u * (uint32_t)wave;
-        const uint32_t lb = lds_addr(sb) + 1024u * (uint32_t)wave;
-#pragma unroll
-        for (int t = 0; t < kDmaPerWave; ++t) {
-            if (t < kATs)
-                dma16(rx, la + 4096u * t, voff[t]);
-            else
-                dma16(rw, lb + 4096u * (t - kATs), voff[t]);
-        }
+        const bool in = kt < KT;
+        rx = rsrc_words(reinterpret_cast<const char*>(xb) + (in ? k0b : 0u),
+                                    in ? rows_x * row_bytes - k0b : 0u);
+        rw = rsrc_words(reinterpret_cast<const char*>(wb) + (in ? k0b : 0u),
+                                    in ? rows_w * row_bytes - k0b : 0u);
+        la = lds0 + buf * kStage;
+    };
+    auto copy = [&](int t) __attribute__((always_inline)) {
+        if (t < kATs)
+            dma16(rx, la + 4096u * t, voff[t]);
+        else
+            dma16(rw, la + kStageA + 4096u * (t - kATs), voff[t]);
     };
 
     f32x16 acc[WMT][2];
@@ -166,7 +166,9 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     const uint32_t a_row0 = (uint32_t)wm * 32u * WMT + n;
     const uint32_t b_row0 = 32u * (uint32_t)wn + n;
 
-    auto compute = [&](const f16* sa, const f16* sb) {
+    auto compute = [&](uint32_t stage_buf) {
+        const f16* sa = lds + stage_buf * (kStage / 2u);
+        const f16* sb = sa + kStageA / 2u;
         f16x8 af[2][WMT], bf[2][2];
         auto fetch = [&](int ks, int buf) {
             const uint32_t pos = 8u * (((uint32_t)(2 * ks) + hh) ^ sw);
@@ -178,64 +180,66 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
                 bf[buf][nt] = lds16(sb + (b_row0 + 64u * nt) * kRowH + pos);
         };
         fetch(0, 0);
+        // the operand reads of k-step ks + 1 stand before the MFMAs of k-step
+        // ks, and the copies of the target stage between the MFMAs: a copy
+        // waits at issue for the ones before it, which leaves the matrix cores
+        // idle where all of a stage's are issued together (256 x 128 tiles:
+        // 38.5 -> 34.8 us at 2500 tokens, 70.4 -> 65.5 at 4100; the smaller
+        // tiles, bound by the copies themselves, run alike)
+        constexpr int kMfmas = 2 * WMT * (kBK / 16);
 #pragma unroll
         for (int ks = 0; ks < kBK / 16; ++ks) {
             const int cur = ks & 1;
             if (ks + 1 < kBK / 16) fetch(ks + 1, cur ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int mt = 0; mt < WMT; ++mt)
+            for (int i = 0; i < 2 * WMT; ++i) {
+                acc[i >> 1][i & 1] = mfma32(af[cur][i >> 1], bf[cur][i & 1], acc[i >> 1][i & 1]);
+                // copies t with t * kMfmas / kDmaPerWave = this MFMA's index
+                const int at = ks * 2 * WMT + i;
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt)
-                    acc[mt][nt] = mfma32(af[cur][mt], bf[cur][nt], acc[mt][nt]);
-        }
-        // schedule: the operand reads of k-step ks + 1 interleaved with the
-        // MFMAs of k-step ks, so one wave per SIMD keeps the MFMA pipe fed
-        // while its LDS reads are in flight
-        constexpr int kReads = WMT + 2, kMfmas = 2 * WMT;
-        __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
-#pragma unroll
-        for (int ks = 0; ks + 1 < kBK / 16; ++ks) {
-#pragma unroll
-            for (int i = 0; i < (kReads > kMfmas ? kReads : kMfmas); ++i) {
-                if (i < kMfmas) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                if (i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                for (int t = 0; t < kDmaPerWave; ++t)
+                    if (t * kMfmas / kDmaPerWave == at) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        copy(t);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
             }
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, kMfmas, 0);
     };
 
-    // stage kt sits in buffer kt % 3; at the top of step kt this wave has
-    // stages kt and kt + 1 in flight: wait for kt, then the barrier makes
-    // every wave's copy of it visible and frees buffer (kt + 2) % 3 (last
-    // read in step kt - 1) for the DMA of stage kt + 2
-    const uint32_t KT = K / kBK;
-    if (KT > 0) stage(0, sa0, sb0);
-    if (KT > 1) stage(1, sa1, sb1);
-    // (a bare s_barrier: __syncthreads' fence would also wait for stage kt + 1)
-    auto step = [&](uint32_t kt, const f16* sa, const f16* sb, f16* na, f16* nb) {
+    // stage kt sits in buffer kt % kStages; at the top of step kt this wave has
+    // stages kt .. kt + kStages - 2 in flight: wait for kt, then the barrier
+    // makes every wave's copy of it visible and frees the buffer read in step
+    // kt - 1 for the DMA of stage kt + kStages - 1
+    // (a bare s_barrier: __syncthreads' fence would also wait for later stages)
+#pragma unroll
+    for (uint32_t kt = 0; kt + 1 < kStages; ++kt) {
+        target(kt, kt);
+#pragma unroll
+        for (int t = 0; t < kDmaPerWave; ++t) copy(t);
+    }
+    uint32_t buf = 0, next = kStages - 1;
+    for (uint32_t kt = 0; kt < KT; ++kt) {
         asm volatile("" ::: "memory");
-        if (kt + 1 < KT)
-            __builtin_amdgcn_s_waitcnt(kWaitOne);
-        else
-            __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_s_waitcnt(kWaitOne);
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (kt + 2 < KT) stage(kt + 2, na, nb);
-        compute(sa, sb);
-    };
-    for (uint32_t kt = 0; kt < KT; kt += 3) {
-        step(kt, sa0, sb0, sa2, sb2);
-        if (kt + 1 < KT) step(kt + 1, sa1, sb1, sa0, sb0);
-        if (kt + 2 < KT) step(kt + 2, sa2, sb2, sa1, sb1);
+        target(kt + kStages - 1, next);
+        compute(buf);
+        next = buf;
+        buf = buf + 1 == kStages ? 0 : buf + 1;
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // the zero stages, before the LDS is written again
 
     // ---- epilogue.  acc[mt][nt][r] is token m0 + wm*32*WMT + 32 mt + 8 (r / 4)
     // + 4 hh + r % 4, feature n0 + 64 nt + c with c = 32 wn + n.  The fp16
-    // tile goes through LDS (features 0..63 in sa0, 64..127 in sa1, both
+    // tile goes through LDS (features 0..63 at sa0, 64..127 at sa1, both
     // [BM][64]) so that every global store is 16 bytes: 8 threads per token
     // row, thread j holding features 8j..8j+7 and 64+8j..64+8j+7 -- the two
     // halves of 8 rotation pairs.
     const uint32_t c = 32u * (uint32_t)wn + n;
+    f16 *sa0 = lds, *sa1 = lds + BM * 64;
     __syncthreads();  // every wave is done with the stage buffers
 #pragma unroll
     for (int mt = 0; mt < WMT; ++mt)
@@ -313,13 +317,13 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     }
 }
 
-// Wide tile for long prompts: a workgroup computes 256 tokens x 384 features
-// (three heads when D = 128) with 8 waves as 2 (tokens) x 4 (features), each
-// wave 128 x 96 on v_mfma_f32_32x32x16_f16, so every X and W byte staged in
-// LDS feeds 1.5x (X) and 3x (W) the MFMA work of the 256 x 128 tile and the
-// X re-reads from L2 drop by two thirds.  64 k-values per stage (128-byte
+// Wide tiles for long prompts: a workgroup computes 256 tokens x 128 NT features
+// (NT heads when D = 128, NT = 3 or 2) with 8 waves as 2 (tokens) x 4
+// (features), each wave 128 x 32 NT on v_mfma_f32_32x32x16_f16, so every X and W byte staged in
+// LDS feeds more MFMA work than in the 256 x 128 tile (NT = 3: X 1.5x and W 3x)
+// and the X re-reads from L2 drop to 1 / NT.  64 k-values per stage (128-byte
 // LDS rows, chunk c of row r at position c ^ ((r >> 1) & 7): conflict-free
-// operand reads), two stages of 80 KiB (all of the LDS; the DMA of stage
+// operand reads), two stages (NT = 3: 80 KiB each, all of the LDS; the DMA of stage
 // kt + 1 runs under the MFMAs of stage kt; 6 % faster than three stages of
 // 32 k-values, which need twice the barriers).  Each output sums its 16-value
 // k-chunks in the same order as qkv_gemm_mfma, so the two kernels give
@@ -327,18 +331,17 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
 // The epilogue runs one head at a time through LDS with the qkv_gemm_mfma
 // store pattern.
 constexpr int kWBM = 256;
-constexpr int kWBN = 384;
 constexpr int kWBK = 64;
 constexpr int kWThreads = 512;
 constexpr int kWADma = kWBM * 8 / 64;                  // 1 KiB DMA instructions per X stage (32)
-constexpr int kWBDma = kWBN * 8 / 64;                  // ... per W stage (48)
 constexpr int kWATs = kWADma / 8;                      // X instructions per wave (4)
-constexpr int kWDmaPerWave = (kWADma + kWBDma) / 8;    // 10
 constexpr uint32_t kWStageA = kWBM * kWBK * 2;         // bytes of X per stage
-constexpr uint32_t kWStage = kWStageA + kWBN * kWBK * 2;  // bytes per stage (80 KiB)
 
-template <bool FUSED>
+template <int NT, bool FUSED>
 __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
+    constexpr int kWBN = 128 * NT;
+    constexpr int kWDmaPerWave = (kWADma + kWBN * 8 / 64) / 8;
+    constexpr uint32_t kWStage = kWStageA + kWBN * kWBK * 2;  // bytes per stage
     __shared__ __attribute__((aligned(16))) f16 lds[2 * kWStage / 2];
 
     const int tid = threadIdx.x;
@@ -355,7 +358,7 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
     const uint32_t K = a.K;
     const uint32_t row_bytes = K * 2u;
     const uint32_t rows_x = a.M - m0;   // >= 1
-    const uint32_t rows_w = a.N - n0;   // = 384 (N is a multiple of 384)
+    const uint32_t rows_w = a.N - n0;   // >= 128 NT (N is a multiple)
     const f16* xb = a.x + (uint64_t)m0 * K;
     const f16* wb = a.w + (uint64_t)n0 * K;
 
@@ -388,17 +391,17 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
         }
     };
 
-    f32x16 acc[4][3];
+    f32x16 acc[4][NT];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 3; ++nt) acc[mt][nt] = f32x16{};
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x16{};
 
-    // operand rows: X rows 128 wm + 32 mt + n, W rows 96 wn + 32 nt + n; both
+    // operand rows: X rows 128 wm + 32 mt + n, W rows 32 NT wn + 32 nt + n; both
     // start at a multiple of 32 plus n, so the swizzle is (n >> 1) & 7
     const uint32_t sw = (n >> 1) & 7u;
     const uint32_t a_row0 = 128u * (uint32_t)wm + n;
-    const uint32_t b_row0 = 96u * (uint32_t)wn + n;
+    const uint32_t b_row0 = 32u * NT * (uint32_t)wn + n;
 
     auto compute = [&](uint32_t kt) {
         const f16* sa = lds + (kt & 1u) * (kWStage / 2u);
@@ -406,15 +409,15 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
 #pragma unroll
         for (int ks = 0; ks < kWBK / 16; ++ks) {
             const uint32_t pos = 8u * (((uint32_t)(2 * ks) + hh) ^ sw);
-            f16x8 af[4], bf[3];
+            f16x8 af[4], bf[NT];
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) af[mt] = lds16(sa + (a_row0 + 32u * mt) * kWBK + pos);
 #pragma unroll
-            for (int nt = 0; nt < 3; ++nt) bf[nt] = lds16(sb + (b_row0 + 32u * nt) * kWBK + pos);
+            for (int nt = 0; nt < NT; ++nt) bf[nt] = lds16(sb + (b_row0 + 32u * nt) * kWBK + pos);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-                for (int nt = 0; nt < 3; ++nt) acc[mt][nt] = mfma32(af[mt], bf[nt], acc[mt][nt]);
+                for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = mfma32(af[mt], bf[nt], acc[mt][nt]);
         }
     };
 
@@ -434,7 +437,7 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
 
     // ---- epilogue, one head (128 features) per round.  acc[mt][nt][r] is
     // token m0 + 128 wm + 32 mt + 8 (r / 4) + 4 hh + r % 4, tile feature
-    // f = 96 wn + 32 nt + n; a 32-feature block never straddles two heads.
+    // f = 32 NT wn + 32 nt + n; a 32-feature block never straddles two heads.
     f16* lo = lds;             // [256][64]: features 0..63 of the round's head
     f16* hi = lds + kWBM * 64; // [256][64]: features 64..127
     const uint32_t N = a.N;
@@ -442,11 +445,11 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
     const uint32_t Hq = a.num_heads, Hkv = a.num_kv_heads;
     const uint64_t kv_dim = (uint64_t)Hkv * 128u;
 #pragma unroll 1
-    for (uint32_t h = 0; h < 3; ++h) {
+    for (uint32_t h = 0; h < NT; ++h) {
         __syncthreads();  // the stages (h = 0) or the previous round's tile are free
 #pragma unroll
-        for (int nt = 0; nt < 3; ++nt) {
-            const uint32_t fb = 96u * (uint32_t)wn + 32u * (uint32_t)nt;  // block's first feature
+        for (int nt = 0; nt < NT; ++nt) {
+            const uint32_t fb = 32u * NT * (uint32_t)wn + 32u * (uint32_t)nt;  // block's first feature
             if (fb / 128u != h) continue;
             const uint32_t c = (fb & 127u) + n;
             f16* dst = (c < 64u ? lo : hi) + (c & 63u);
@@ -542,29 +545,61 @@ hipError_t launch_mfma(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <int NT>
 hipError_t launch_wide(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
     QkvGemmArgs b = a;
-    b.n_tiles = a.N / kWBN;
+    b.n_tiles = a.N / (128u * NT);
     b.vec_out = 1u;
     b.m_tiles = (a.M + kWBM - 1u) / kWBM;
     const uint64_t blocks = (uint64_t)b.m_tiles * b.n_tiles;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     if (fused)
-        hipLaunchKernelGGL(qkv_gemm_wide<true>, dim3((uint32_t)blocks), dim3(kWThreads), 0, stream,
-                           b);
+        hipLaunchKernelGGL((qkv_gemm_wide<NT, true>), dim3((uint32_t)blocks), dim3(kWThreads), 0,
+                           stream, b);
     else
-        hipLaunchKernelGGL(qkv_gemm_wide<false>, dim3((uint32_t)blocks), dim3(kWThreads), 0, stream,
-                           b);
+        hipLaunchKernelGGL((qkv_gemm_wide<NT, false>), dim3((uint32_t)blocks), dim3(kWThreads), 0,
+                           stream, b);
     return hipGetLastError();
 }
 
-// The wide tile needs whole 384-feature tiles and 16-byte aligned output
-// rows; it pays off once there are enough token tiles to fill the CUs.
-bool use_wide(const QkvGemmArgs& a) {
-    const long forced = get_option(kOptQkvGemmWide);
-    if (forced == 1) return false;
-    if (a.N % kWBN != 0 || a.K % kWBK != 0 || !aligned16(a.y)) return false;
-    return forced == 2 || a.M >= kWideMinTokens;
+// Tiles in the order of their rows: the cost of one round of workgroups (one
+// per CU) in tenths of a microsecond at K = 2048, measured with the weights in
+// the memory-side cache and a part of the CUs busy; all scale with K.
+struct Tile {
+    uint32_t tokens, features, cost;
+};
+constexpr Tile kTiles[] = {
+    {64, 128, 130}, {128, 128, 165}, {256, 128, 250}, {256, 256, 460}, {256, 384, 660}};
+
+// The tile whose rounds cost least.  All tiles add a feature's k-values in the
+// same order, so the choice never shows in the results.  N = 3072, us for 64 x
+// 128 / 128 x 128 / 256 x 128 / 256 x 256 / 256 x 384 tiles: 512 tokens 13.1 /
+// 15.9 / 24.4, 999 21.4 / 18.6 / 25.6, 1280 24.2 / 20.0 / 25.7, 2500 - / 39.5 /
+// 33.7 / 47.4, 2600 - / 40.0 / 54.7 / 47.9, 4100 - / 68.6 / 59.3 / 54.6 / 68.5,
+// 5200 - / 75.8 / 68.1 / 64.0 / 73.6, 6400 - / 90.4 / 93.0 / 104.9 / 84.4, 8192
+// - / 110 / 99.9 / 107 / 92.1.
+int pick_tile(const QkvGemmArgs& a, int device) {
+    const long forced = get_option(kOptQkvGemmTokensPerWave), wide = get_option(kOptQkvGemmWide);
+    const auto wide_fits = [&](uint32_t features) {
+        return a.N % features == 0 && a.K % kWBK == 0 && aligned16(a.y);
+    };
+    if (wide == 2 && wide_fits(384)) return 4;
+    if (forced == 32 || forced == 64 || forced == 128) return forced == 32 ? 0 : forced == 64 ? 1 : 2;
+    const uint64_t cus = (uint64_t)device_cu_count(device);
+    int best = -1;
+    uint64_t least = 0;
+    for (int i = 0; i < 5; ++i) {
+        const Tile& t = kTiles[i];
+        if (i >= 3 && (wide == 1 || !wide_fits(t.features))) continue;
+        const uint64_t wgs = (uint64_t)((a.M - 1u) / t.tokens + 1u) *
+                             ((a.N - 1u) / t.features + 1u);
+        const uint64_t cost = (wgs + cus - 1) / cus * t.cost;
+        if (best < 0 || cost < least) {
+            best = i;
+            least = cost;
+        }
+    }
+    return best;
 }
 
 }  // namespace
@@ -574,12 +609,6 @@ bool qkv_gemm_mfma_ok(const QkvGemmArgs& a) {
     if (a.K % kBK != 0 || !aligned16(a.x) || !aligned16(a.w)) return false;
     // every row offset of X and W fits the 32-bit buffer ranges
     return (uint64_t)a.M * a.K * 2u < 0xffffffffull && (uint64_t)a.N * a.K * 2u < 0xffffffffull;
-}
-
-int qkv_gemm_wmt(uint32_t M) {
-    const long forced = get_option(kOptQkvGemmTokensPerWave);
-    if (forced == 32 || forced == 64 || forced == 128) return (int)(forced / 32);
-    return M > 1024u ? 4 : (M > 256u ? 2 : 1);
 }
 
 hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
@@ -593,15 +622,16 @@ hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t 
         hipLaunchKernelGGL(qkv_gemm_generic, dim3((uint32_t)blocks), dim3(256), 0, stream, b);
         return hipGetLastError();
     }
-    if (use_wide(a)) return launch_wide(a, fused, stream);
     int device = 0;
     if (hipError_t e = hipGetDevice(&device)) return e;
     if (const int tile = qkv_short_tile(a, device); tile >= 0)
         return launch_qkv_gemm_short(a, tile, fused, stream);
-    switch (qkv_gemm_wmt(a.M)) {
-        case 1: return launch_mfma<1>(a, fused, stream);
-        case 2: return launch_mfma<2>(a, fused, stream);
-        default: return launch_mfma<4>(a, fused, stream);
+    switch (pick_tile(a, device)) {
+        case 0: return launch_mfma<1>(a, fused, stream);
+        case 1: return launch_mfma<2>(a, fused, stream);
+        case 2: return launch_mfma<4>(a, fused, stream);
+        case 3: return launch_wide<2>(a, fused, stream);
+        default: return launch_wide<3>(a, fused, stream);
     }
 }
 

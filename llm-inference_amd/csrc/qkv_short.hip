@@ -286,7 +286,9 @@ constexpr Tile kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {32, 16}, {16, 16}};
 // Up to 256 tokens: beyond, the tiles add k-values in one order whatever their
 // size.  Below K = 1024 a wave has two units or less, nothing for a ring.
 int qkv_short_tile(const QkvGemmArgs& a, int device) {
-    if (a.M > 256u || a.K < 1024u || get_option(kOptQkvGemmTokensPerWave)) return -1;
+    if (a.M > 256u || a.K < 1024u || get_option(kOptQkvGemmTokensPerWave) ||
+        get_option(kOptQkvGemmWide) == 2)
+        return -1;
     const uint64_t cus = (uint64_t)device_cu_count(device);
     int best = -1;
     uint64_t least = 0;
