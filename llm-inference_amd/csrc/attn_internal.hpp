@@ -56,9 +56,9 @@ struct QkvGemmArgs {
     const f16* x;        // [M][K]
     const f16* w;        // [N][K]: Q rows, then K, then V
     f16* y;              // [M][N] (fused: Q rotated, K and V as projected)
-    f16* kc;             // fused: K cache rows [S][Hkv*128]
+    f16* kc;             // fused: K cache rows [S][Hkv*D]
     f16* vc;             // fused: V cache rows
-    const f16* cos_t;    // fused: [S][64]
+    const f16* cos_t;    // fused: [S][D/2]
     const f16* sin_t;
     uint32_t M;
     uint32_t N;
@@ -66,6 +66,7 @@ struct QkvGemmArgs {
     uint32_t n_tiles;    // set by the launcher
     uint32_t num_heads;
     uint32_t num_kv_heads;
+    uint32_t head_dim;   // fused: 128, or 64 (not the short-prompt kernels)
     uint32_t start_pos;  // fused: cache/table row of token 0
     uint32_t apply;      // fused: 1 rotate Q and K, 0 NoPE
     uint32_t vec_out;    // set by the launcher: 16-byte stores of y (N % 8 == 0, y aligned)

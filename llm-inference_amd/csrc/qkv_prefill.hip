@@ -81,6 +81,56 @@ __device__ __forceinline__ void map_tile(uint32_t bid, uint32_t m_tiles, uint32_
     }
 }
 
+// One thread's columns of a fused tile of 128 features staged as [rows][64]
+// twice, features 0..63 and 64..127: 8 rotation pairs of a head, with the
+// destinations of the halves.  D = 128: the tile is one head, pairs (c, c + 64);
+// D = 64: two heads, threads 0-3 of a row the first, pairs (c, c + 32).
+struct FusedCols {
+    uint32_t head, half;        // half = D / 2
+    uint32_t tcol;              // column of the first half, in the head and the table
+    uint32_t col;               // ... in the tile
+    uint32_t lo, hi;            // staged halves
+    bool is_q, rot;
+    f16* cache;
+    uint64_t kv_dim;
+    __device__ __forceinline__ FusedCols(const QkvGemmArgs& a, uint32_t tile, uint32_t j8,
+                                         uint32_t rows) {
+        const bool d64 = a.head_dim == 64u;
+        const uint32_t second = d64 ? j8 >> 5 : 0u;
+        half = d64 ? 32u : 64u;
+        head = d64 ? 2u * tile + second : tile;
+        tcol = d64 ? j8 & 31u : j8;
+        col = 64u * second + tcol;
+        lo = second * rows * 64u + tcol;
+        hi = d64 ? lo + 32u : rows * 64u + j8;
+        const uint32_t Hq = a.num_heads, Hkv = a.num_kv_heads;
+        is_q = head < Hq;
+        const bool is_k = !is_q && head < Hq + Hkv;
+        rot = a.apply != 0 && (is_q || is_k);
+        kv_dim = (uint64_t)Hkv * a.head_dim;
+        cache = is_q ? nullptr
+                     : (is_k ? a.kc + (uint64_t)(head - Hq) * a.head_dim
+                             : a.vc + (uint64_t)(head - Hq - Hkv) * a.head_dim);
+    }
+    __device__ __forceinline__ void store(const QkvGemmArgs& a, const f16* staged, uint32_t m,
+                                          uint32_t n0, f16x8 cs, f16x8 sn) const {
+        const f16x8 x0 = lds16(staged + lo), x1 = lds16(staged + hi);
+        f16x8 r0 = x0, r1 = x1;
+        if (rot) rope_rotate8(x0, x1, cs, sn, r0, r1);
+        f16* yr = a.y + (uint64_t)m * a.N + n0 + col;
+        if (is_q) {
+            st16(yr, r0);
+            st16(yr + half, r1);
+        } else {
+            st16(yr, x0);
+            st16(yr + half, x1);
+            f16* cr = cache + ((uint64_t)a.start_pos + m) * kv_dim + tcol;
+            st16(cr, r0);
+            st16(cr + half, r1);
+        }
+    }
+};
+
 template <int WMT, bool FUSED>
 __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     constexpr int BM = 64 * WMT;
@@ -273,23 +323,17 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
         }
         return;
     }
-    // fused: the tile is head n_tile (D = 128, N = (Hq + 2 Hkv) * 128)
-    const uint32_t head = n_tile;
-    const uint32_t Hq = a.num_heads, Hkv = a.num_kv_heads;
-    const uint64_t kv_dim = (uint64_t)Hkv * 128u;
-    const bool is_q = head < Hq;
-    const bool is_k = !is_q && head < Hq + Hkv;
-    const bool rot = a.apply != 0 && (is_q || is_k);
-    f16* cache = is_q ? nullptr
-                      : (is_k ? a.kc + (uint64_t)(head - Hq) * 128u
-                              : a.vc + (uint64_t)(head - Hq - Hkv) * 128u);
+    // fused: the tile is head n_tile (D = 128) or heads 2 n_tile and 2 n_tile + 1
+    // (D = 64; the second may lie past N)
+    const FusedCols f(a, n_tile, j8, BM);
+    if (f.head >= a.num_heads + 2u * a.num_kv_heads) return;
     // table rows of all passes first (rows past M read row M - 1, unused)
     f16x8 cs[BM / 32], sn[BM / 32];
-    if (rot) {
+    if (f.rot) {
 #pragma unroll
         for (int p = 0; p < BM / 32; ++p) {
             const uint32_t m = min(m0 + 32u * p + rsub, a.M - 1u);
-            const uint64_t t = ((uint64_t)a.start_pos + m) * 64u + j8;
+            const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
             cs[p] = ld16(a.cos_t + t);
             sn[p] = ld16(a.sin_t + t);
         }
@@ -298,22 +342,7 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     for (int p = 0; p < BM / 32; ++p) {
         const uint32_t row = 32u * p + rsub, m = m0 + row;
         if (m >= a.M) break;
-        const f16x8 lo = lds16(sa0 + row * 64u + j8);
-        const f16x8 hi = lds16(sa1 + row * 64u + j8);
-        f16x8 r0 = lo, r1 = hi;
-        if (rot) rope_rotate8(lo, hi, cs[p], sn[p], r0, r1);
-        f16* yr = a.y + (uint64_t)m * N + n0;
-        const uint64_t pos = (uint64_t)a.start_pos + m;
-        if (is_q) {
-            st16(yr + j8, r0);
-            st16(yr + 64u + j8, r1);
-        } else {
-            st16(yr + j8, lo);
-            st16(yr + 64u + j8, hi);
-            f16* cr = cache + pos * kv_dim;
-            st16(cr + j8, r0);
-            st16(cr + 64u + j8, r1);
-        }
+        f.store(a, lds + row * 64u, m, n0, cs[p], sn[p]);
     }
 }
 
@@ -442,8 +471,6 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
     f16* hi = lds + kWBM * 64; // [256][64]: features 64..127
     const uint32_t N = a.N;
     const uint32_t j8 = 8u * ((uint32_t)tid & 7u), rsub = (uint32_t)tid >> 3;
-    const uint32_t Hq = a.num_heads, Hkv = a.num_kv_heads;
-    const uint64_t kv_dim = (uint64_t)Hkv * 128u;
 #pragma unroll 1
     for (uint32_t h = 0; h < NT; ++h) {
         __syncthreads();  // the stages (h = 0) or the previous round's tile are free
@@ -475,38 +502,19 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
             }
             continue;
         }
-        // fused: the round's tile is head hn0 / 128 (D = 128)
-        const uint32_t head = hn0 / 128u;
-        const bool is_q = head < Hq;
-        const bool is_k = !is_q && head < Hq + Hkv;
-        const bool rot = a.apply != 0 && (is_q || is_k);
-        f16* cache = is_q ? nullptr
-                          : (is_k ? a.kc + (uint64_t)(head - Hq) * 128u
-                                  : a.vc + (uint64_t)(head - Hq - Hkv) * 128u);
+        // fused: the round's tile is head hn0 / 128 (D = 128) or two heads (D = 64)
+        const FusedCols f(a, hn0 / 128u, j8, kWBM);
 #pragma unroll
         for (int p = 0; p < kWBM / 64; ++p) {
             const uint32_t row = 64u * p + rsub, m = m0 + row;
             if (m >= a.M) break;
-            const f16x8 x0 = lds16(lo + row * 64u + j8);
-            const f16x8 x1 = lds16(hi + row * 64u + j8);
-            f16x8 r0 = x0, r1 = x1;
-            const uint64_t pos = (uint64_t)a.start_pos + m;
-            if (rot) {
-                const f16x8 cs = ld16(a.cos_t + pos * 64u + j8);
-                const f16x8 sn = ld16(a.sin_t + pos * 64u + j8);
-                rope_rotate8(x0, x1, cs, sn, r0, r1);
+            f16x8 cs{}, sn{};
+            if (f.rot) {
+                const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
+                cs = ld16(a.cos_t + t);
+                sn = ld16(a.sin_t + t);
             }
-            f16* yr = a.y + (uint64_t)m * N + hn0;
-            if (is_q) {
-                st16(yr + j8, r0);
-                st16(yr + 64u + j8, r1);
-            } else {
-                st16(yr + j8, x0);
-                st16(yr + 64u + j8, x1);
-                f16* cr = cache + pos * kv_dim;
-                st16(cr + j8, r0);
-                st16(cr + 64u + j8, r1);
-            }
+            f.store(a, lds + row * 64u, m, hn0, cs, sn);
         }
     }
 }

@@ -45,3 +45,23 @@ def test_automatic_tile_fused_bitexact(attn, gpu, M, start_pos, rotate):
     print(f"[case] fused tiles M={M} pos={start_pos} rotate={rotate}", flush=True)
     fy, fc, ty, tc, _ = fused_case(attn, gpu, M, start_pos, rotate, K=192)
     assert np.array_equal(fy, ty) and np.array_equal(fc, tc)
+
+
+# head_dim 64: two heads to a 128-feature tile, the last one alone where
+# Hq + 2 Hkv is odd; each tile; both sides of the short prompts
+@pytest.mark.parametrize("Hq,Hkv", [(16, 4), (3, 1), (5, 1), (8, 8)])
+@pytest.mark.parametrize("M,start_pos,rotate", [(256, 0, True), (257, 9, True), (1300, 3, False),
+                                                (3333, 2, True), (6000, 0, True)])
+def test_fused_64_dim_heads_bitexact(attn, gpu, Hq, Hkv, M, start_pos, rotate):
+    print(f"[case] fused d64 {Hq}/{Hkv} M={M} pos={start_pos} rotate={rotate}", flush=True)
+    fy, fc, ty, tc, _ = fused_case(attn, gpu, M, start_pos, rotate, Hq, Hkv, 64, 192)
+    assert np.array_equal(fy, ty) and np.array_equal(fc, tc)
+
+
+def test_fused_64_dim_heads_wide_tile(attn, gpu):
+    try:
+        attn.set_option("qkv_gemm_wide", 2)
+        fy, fc, ty, tc, _ = fused_case(attn, gpu, 700, 5, True, 16, 4, 64, 192)
+    finally:
+        attn.set_option("qkv_gemm_wide", 0)
+    assert np.array_equal(fy, ty) and np.array_equal(fc, tc)
