@@ -262,7 +262,8 @@ int attn_qkv_gemm(const attn_f16_t* x, attn_f16_t* y, const attn_f16_t* w, size_
  * launch_rope_and_store_kv(y, y + Hq*D, y + (Hq+Hkv)*D, k_cache, v_cache, cos,
  * sin, seq_len, Hq, Hkv, D, total, total, start_pos, apply_rotation) -- the
  * pair ModelInference issues back to back in prefill (model_inference.hpp:
- * 266-285) -- as one kernel when head_dim == 128, the GEMM takes its MFMA
+ * 266-285) -- as one kernel when head_dim == 128 (or 64 with more than 256
+ * tokens), the GEMM takes its MFMA
  * path and y, the caches and the tables are 16-byte aligned (the two launches
  * otherwise).  Results equal attn_qkv_gemm followed by
  * attn_rope_store_kv bit for bit. */
@@ -372,9 +373,9 @@ int attn_prefill_plan(const void* q, const void* k, const void* v, const void* o
  * kernel reads K in whole 256-byte rows through LDS-DMA, otherwise straight
  * into registers; 1 = registers, 2 = LDS-DMA), "prefill_force_generic",
  * "qkv_gemm_force_generic", "qkv_gemm_tokens_per_wave" (0 = automatic; 32, 64
- * or 128 tokens per wave of the 256 x 128-tile MFMA GEMM), "qkv_gemm_wide"
- * (0 = automatic, by the rounds of workgroups; 1 = never; 2 = whenever N is a multiple
- * of 384 and Y is 16-byte aligned), "prefill_waves" (0 = automatic: 4-wave
+ * or 128 tokens per wave of the 128-feature MFMA GEMM tiles), "qkv_gemm_wide"
+ * (0 = automatic, by the rounds of workgroups; 1 = never; 2 = the 256 x 384
+ * tile whenever N is a multiple of 384 and Y is 16-byte aligned), "prefill_waves" (0 = automatic: 4-wave
  * workgroups of 32 queries up to 6144 tokens, 8-wave workgroups of 64 queries
  * above; 4 or 8 forces one), "prefill_stage_all" (0 = automatic: up to 256
  * tokens every key tile of a 4-wave workgroup is copied into LDS at once;
