@@ -262,8 +262,7 @@ int attn_qkv_gemm(const attn_f16_t* x, attn_f16_t* y, const attn_f16_t* w, size_
  * launch_rope_and_store_kv(y, y + Hq*D, y + (Hq+Hkv)*D, k_cache, v_cache, cos,
  * sin, seq_len, Hq, Hkv, D, total, total, start_pos, apply_rotation) -- the
  * pair ModelInference issues back to back in prefill (model_inference.hpp:
- * 266-285) -- as one kernel when head_dim == 128 (or 64 with more than 256
- * tokens), the GEMM takes its MFMA
+ * 266-285) -- as one kernel when head_dim is 128 or 64, the GEMM takes its MFMA
  * path and y, the caches and the tables are 16-byte aligned (the two launches
  * otherwise).  Results equal attn_qkv_gemm followed by
  * attn_rope_store_kv bit for bit. */

@@ -512,11 +512,11 @@ int attn_qkv_gemm_rope_store_kv(const attn_f16_t* x, attn_f16_t* y, const attn_f
     QkvGemmArgs a;
     if (int rc = qkv_gemm_args(a, x, y, w, seq_len, hidden_size, total)) return rc;
     const auto a16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
-    // head_dim 64 from 257 tokens (the short prompts' tiles hold no whole pairs of
-    // it): two launches against one, 16/4 heads, us: 300 tokens 15.7 / 12.5, 1500
-    // 22.1 / 19.1, 4096 37.2 / 32.9
-    if ((head_dim == 128 || (head_dim == 64 && seq_len > 256)) && qkv_gemm_mfma_ok(a) &&
-        a16(y) && a16(k_cache) && a16(v_cache) && a16(cos_table) && a16(sin_table)) {
+    // two launches against one at head_dim 64, 16/4 heads, us: 24 tokens 8.8 /
+    // 5.1, 100 10.0 / 6.3, 256 11.6 / 8.2, 300 15.7 / 12.5, 1500 22.1 / 19.1, 4096
+    // 37.2 / 32.9
+    if ((head_dim == 128 || head_dim == 64) && qkv_gemm_mfma_ok(a) && a16(y) && a16(k_cache) &&
+        a16(v_cache) && a16(cos_table) && a16(sin_table)) {
         a.kc = reinterpret_cast<f16*>(k_cache);
         a.vc = reinterpret_cast<f16*>(v_cache);
         a.cos_t = reinterpret_cast<const f16*>(cos_table);

@@ -66,7 +66,7 @@ struct QkvGemmArgs {
     uint32_t n_tiles;    // set by the launcher
     uint32_t num_heads;
     uint32_t num_kv_heads;
-    uint32_t head_dim;   // fused: 128, or 64 (not the short-prompt kernels)
+    uint32_t head_dim;   // fused: 64 or 128
     uint32_t start_pos;  // fused: cache/table row of token 0
     uint32_t apply;      // fused: 1 rotate Q and K, 0 NoPE
     uint32_t vec_out;    // set by the launcher: 16-byte stores of y (N % 8 == 0, y aligned)

@@ -13,7 +13,8 @@
 //    rounds of workgroups times the rows of a tile are least
 //    (qkv_short_tile): 128 instead of 192 rows per workgroup at 254 tokens, 48
 //    at 24.  A tile's features are BN/2 columns of a head and the same columns
-//    + 64, so both halves of every rotation pair are in the workgroup.
+//    + D / 2, so both halves of every rotation pair are in the workgroup (not
+//    fused: as for D = 128).
 //  * the waves split K: wave w takes the 64-value units w, w + W, ... with a
 //    ring of copies (buffer_load ... lds) of its own, computes the whole tile
 //    for them, and the W fp32 tiles are added through LDS at the end, in wave
@@ -78,14 +79,15 @@ __global__ __launch_bounds__(64 * W, 1) void qkv_gemm_short(QkvGemmArgs a) {
     }
     mt0 = __builtin_amdgcn_readfirstlane(mt0);
     nt0 = __builtin_amdgcn_readfirstlane(nt0);
-    constexpr uint32_t kPerHead = 64u / kHalf;
-    const uint32_t head = nt0 / kPerHead, c0 = (nt0 - head * kPerHead) * kHalf;
-    const uint32_t m0 = mt0 * BM, n0 = head * 128u;
+    const uint32_t pair = FUSED ? a.head_dim >> 1 : 64u;  // distance of a pair's columns
+    const uint32_t per_head = pair / kHalf;
+    const uint32_t head = nt0 / per_head, c0 = (nt0 - head * per_head) * kHalf;
+    const uint32_t m0 = mt0 * BM, n0 = head * 2u * pair;
     const uint32_t K = a.K, row_bytes = K * 2u;
     const char* xb = reinterpret_cast<const char*>(a.x + (uint64_t)m0 * K);
     const char* wb = reinterpret_cast<const char*>(a.w + (uint64_t)n0 * K);
     const uint32_t x_bytes = min(a.M - m0, (uint32_t)BM) * row_bytes;
-    const uint32_t w_bytes = min(a.N - n0, 128u) * row_bytes;
+    const uint32_t w_bytes = min(a.N - n0, 2u * pair) * row_bytes;
 
     // copy t: tile rows 8 t .. 8 t + 7 (X rows first, then W rows), lane L
     // writes position L % 8 of row L / 8
@@ -98,7 +100,7 @@ __global__ __launch_bounds__(64 * W, 1) void qkv_gemm_short(QkvGemmArgs a) {
             row = 8u * t + lr;
         } else {
             const uint32_t f = 8u * (t - BM / 8) + lr;
-            row = c0 + (f < kHalf ? f : 64u + f - kHalf);
+            row = c0 + (f < kHalf ? f : pair + f - kHalf);
         }
         voff[t] = row * row_bytes +
                   16u * (((uint32_t)lane & 7u) ^ ((4u * (t & 1) + (lr >> 1)) & 7u));
@@ -112,13 +114,13 @@ __global__ __launch_bounds__(64 * W, 1) void qkv_gemm_short(QkvGemmArgs a) {
     const bool is_q = head < Hq, is_k = !is_q && head < Hq + Hkv;
     const bool rot = FUSED && a.apply != 0 && (is_q || is_k);
     const uint32_t erow = (uint32_t)tid / (kHalf / P), ec = ((uint32_t)tid % (kHalf / P)) * P;
-    const uint32_t m = m0 + erow, col = c0 + ec;  // and col + 64
+    const uint32_t m = m0 + erow, col = c0 + ec;  // and col + pair
     const bool mine = erow < (uint32_t)BM && m < a.M;
     const uint64_t pos = (uint64_t)a.start_pos + m;
     hv cs = {}, sn = {};
     if (rot && mine) {
-        cs = *reinterpret_cast<const hv*>(a.cos_t + pos * 64u + col);
-        sn = *reinterpret_cast<const hv*>(a.sin_t + pos * 64u + col);
+        cs = *reinterpret_cast<const hv*>(a.cos_t + pos * pair + col);
+        sn = *reinterpret_cast<const hv*>(a.sin_t + pos * pair + col);
     }
 
     const uint32_t units = K / 64u;
@@ -244,15 +246,15 @@ __global__ __launch_bounds__(64 * W, 1) void qkv_gemm_short(QkvGemmArgs a) {
     }
     if (is_q) {
         *reinterpret_cast<hv*>(yr) = r0;
-        *reinterpret_cast<hv*>(yr + 64) = r1;
+        *reinterpret_cast<hv*>(yr + pair) = r1;
     } else {
         *reinterpret_cast<hv*>(yr) = lo;
-        *reinterpret_cast<hv*>(yr + 64) = hi;
-        f16* cr = (is_k ? a.kc + (uint64_t)(head - Hq) * 128u
-                        : a.vc + (uint64_t)(head - Hq - Hkv) * 128u) +
-                  pos * ((uint64_t)Hkv * 128u) + col;
+        *reinterpret_cast<hv*>(yr + pair) = hi;
+        f16* cr = (is_k ? a.kc + (uint64_t)(head - Hq) * a.head_dim
+                        : a.vc + (uint64_t)(head - Hq - Hkv) * a.head_dim) +
+                  pos * ((uint64_t)Hkv * a.head_dim) + col;
         *reinterpret_cast<hv*>(cr) = r0;
-        *reinterpret_cast<hv*>(cr + 64) = r1;
+        *reinterpret_cast<hv*>(cr + pair) = r1;
     }
 }
 
@@ -260,7 +262,8 @@ template <int BM, int BN, int W, int S, int P>
 hipError_t launch(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
     QkvGemmArgs b = a;
     b.m_tiles = (a.M + BM - 1u) / BM;
-    b.n_tiles = (a.N + 127u) / 128u * (128u / BN);
+    const uint32_t span = fused ? a.head_dim : 128u;  // features whose tiles pair up
+    b.n_tiles = (a.N + span - 1u) / span * (span / BN);
     b.vec_out = (a.N % 8u == 0 && ((uintptr_t)a.y & 15u) == 0) ? 1u : 0u;
     const uint64_t blocks = (uint64_t)b.m_tiles * b.n_tiles;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;

@@ -38,3 +38,15 @@ def test_short_prompt_fused_bitexact(attn, gpu, M, start_pos, rotate, Hq, Hkv):
     fy, fc, ty, tc, _ = fused_case(attn, gpu, M, start_pos, rotate, Hq, Hkv)
     assert np.array_equal(fy, ty), "y"
     assert np.array_equal(fc, tc), "cache"
+
+
+# head_dim 64, an odd and an even number of heads, each tile
+@pytest.mark.parametrize("M,start_pos,rotate", [(1, 5, True), (16, 0, True), (17, 3, False),
+                                                (33, 0, True), (64, 7, True), (97, 1, True),
+                                                (130, 0, True), (256, 9, True)])
+@pytest.mark.parametrize("Hq,Hkv", [(16, 4), (3, 1), (32, 8), (5, 1)])
+def test_short_prompt_fused_64_dim_heads_bitexact(attn, gpu, M, start_pos, rotate, Hq, Hkv):
+    print(f"[case] short fused d64 M={M} pos={start_pos} {Hq}/{Hkv}", flush=True)
+    fy, fc, ty, tc, _ = fused_case(attn, gpu, M, start_pos, rotate, Hq, Hkv, 64, 1024)
+    assert np.array_equal(fy, ty), "y"
+    assert np.array_equal(fc, tc), "cache"
