@@ -44,6 +44,7 @@
 // ~600 cycles for 512 cycles of MFMAs; short prompts are bound by the ~4 us of
 // first copies, code fetch and state fold, long ones by the power the MFMAs draw.
 #include "attn_internal.hpp"
+#include "rows64_copies.hpp"
 
 #include <type_traits>
 #include <utility>
@@ -551,7 +552,6 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
 
     using rK = std::integral_constant<int, 1>;
     using rV = std::integral_constant<int, 2>;
-    using cNI = std::integral_constant<int, NI>;
     auto landed = [](auto n_tag) {  // at most n copies of this wave are in flight
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(n_tag)::value));
@@ -578,11 +578,11 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
         uint32_t ku = KS == 4 ? ring : lds0 + part * 2u * kUnitB;
         uint32_t vu = KS == 4 ? ring + 3u * kUnitB : ku + kUnitB;
         if constexpr (KS == 4) {
-            unit_k();
-            unit_v();
-            unit_k();
-            unit_k();
-            landed(std::integral_constant<int, 3 * NI>{});
+            each<4>([&](auto t) __attribute__((always_inline)) {
+                if constexpr (rows64::kFirst.k[decltype(t)::value]) unit_k();
+                else unit_v();
+            });
+            landed(std::integral_constant<int, rows64::kLeftFirst * NI>{});
         } else {
             stage();
             stage();
@@ -591,7 +591,9 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
             meet();
         }
         // Q has landed too: without this, the compiler waits for it at its first
-        // uses in the loop, and with it, in every iteration, for every copy
+        // uses in the loop, and with it, in every iteration, for every copy.  Its
+        // wait here leaves none of the first copies in flight either (it does not
+        // count them); nothing below relies on that
 #pragma unroll
         for (int s = 0; s < NK; ++s) {
             if constexpr (kAsm) asm volatile("" : "+a"(A.q[s]), "+a"(B.q[s]));
@@ -625,10 +627,11 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                 constexpr int sl = decltype(sl_tag)::value;
                 if constexpr (KS == 4) {
                     // K of unit i has been read: its LDS takes unit i + 3's.  K of
-                    // unit i + 1 has landed; K i + 2, V i + 1 and K i + 3 may be in
-                    // flight
+                    // unit i + 1 has landed; K i + 2, V i and K i + 3 may be in
+                    // flight (rows64_copies.hpp)
                     if constexpr (sl < NC) copy_kt(sl_tag, rk, k_to);
-                    if constexpr (sl == NK - 1) landed(std::integral_constant<int, 3 * NI>{});
+                    if constexpr (sl == NK - 1)
+                        landed(std::integral_constant<int, rows64::kLeftK * NI>{});
                     if constexpr (sl == NC) {
                         advance(sk);
                         rk = resource(sk);
@@ -642,7 +645,8 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                 }
             });
             settle(A, B, unit_of(i), dB);
-            if constexpr (KS == 4) landed(cNI{});  // V of unit i; K i + 3 may be in flight
+            if constexpr (KS == 4)  // V of unit i; K i + 3 may be in flight
+                landed(std::integral_constant<int, rows64::kLeftV * NI>{});
             phase(B, A, rV{}, vu, [&](auto sl_tag) __attribute__((always_inline)) {
                 constexpr int sl = decltype(sl_tag)::value;
                 constexpr int c = sl - ND;  // the slots without operand reads
