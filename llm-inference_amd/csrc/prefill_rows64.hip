@@ -35,7 +35,14 @@
 //    rounded weight and what it leaves, 22 bits together), so the outputs are
 //    as close to float64 as attention_generic's, whose layouts these instances
 //    take over (relative error 2.01e-4 either way at 16/4 heads of 64 and 16/16
-//    of 128, the fp16 rounding of the output; 2.5e-4 without).
+//    of 128, the fp16 rounding of the output; 2.5e-4 without).  Far below the
+//    row's largest weight two halves run out of exponent, which shows where the
+//    large weights meet a V of zero (an attention sink): what is left of weights
+//    14.6 nats and more below is multiplied apart (2.1e-4 either way beside sinks
+//    of 6 to 20 nats; without it 2.9e-4 at 12 and 0.3-0.5 at 20).  Units with such
+//    weights cost 2-3 phases instead of one: 16/16 heads of 128, 1000 tokens 18.7 us
+//    where scores have a deviation of 1, 24 of 2, 47 of 3; 16/4 of 64, 1500 tokens
+//    18.1, 24, 35 (attention_generic 570 and 650).
 // Measured (one MI355X, graphs of 20 calls, us, against attention_generic):
 // 16/4 heads of 64: 500 tokens 8.5 (78), 1500 17.1 (643), 4096 64 (4818);
 // 16/16 heads of 128: 130 tokens 8.6 (18.4), 1000 17.0 (582), 4096 118 (9267);
@@ -59,12 +66,22 @@ constexpr int kUnit = 32;  // keys per unit
 // raised: each stays below the fp16 maximum, and weights that small keys get
 // only gain by a maximum that lags
 constexpr float kSumLimit = 4096.f;
+// LO: weights are 2^kUp times the plain ones (as much as leaves flat scores half of
+// the limit), because fp16 ends at 2^-24: the two halves hold 22 bits of a weight
+// from 2^-3 on and 14 at kSmall.  What they leave of weights below kSmall (14.6 nats
+// under the maximum) is multiplied apart, 2^kUpRest times as large.
+constexpr float kUp = 11.f;
+constexpr float kSumLimitLo = 65000.f;
+constexpr float kSmall = 0x1p-10f;
+constexpr uint16_t kSmallBits = 0x1400;  // as fp16
+constexpr float kUpRest = 0x1p36f;
 // running maximum before the first key: finite, so masked scores (-inf) get
 // weight 0 without a special case
 constexpr float kNoMax = -1.0e30f;
 
 #define LDS_AS __attribute__((address_space(3)))
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -107,6 +124,25 @@ __device__ __forceinline__ void scale_acc4(float& a, float& b, float& c, float& 
         : "+a"(a), "+a"(b), "+a"(c), "+a"(d), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
         : "v"(f));
 }
+// four values kept in accumulation registers plus v times f
+__device__ __forceinline__ void add_acc4(float& a, float& b, float& c, float& d, f32x4 v, float f) {
+    float t0, t1, t2, t3;
+    asm volatile(
+        "v_accvgpr_read_b32 %4, %0\n\t"
+        "v_accvgpr_read_b32 %5, %1\n\t"
+        "v_accvgpr_read_b32 %6, %2\n\t"
+        "v_accvgpr_read_b32 %7, %3\n\t"
+        "v_fma_f32 %4, %8, %12, %4\n\t"
+        "v_fma_f32 %5, %9, %12, %5\n\t"
+        "v_fma_f32 %6, %10, %12, %6\n\t"
+        "v_fma_f32 %7, %11, %12, %7\n\t"
+        "v_accvgpr_write_b32 %0, %4\n\t"
+        "v_accvgpr_write_b32 %1, %5\n\t"
+        "v_accvgpr_write_b32 %2, %6\n\t"
+        "v_accvgpr_write_b32 %3, %7"
+        : "+a"(a), "+a"(b), "+a"(c), "+a"(d), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3)
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(f));
+}
 // LDS reads at a byte address: 16 bytes, and four fp16 of one column
 // (ds_read_b64_tr_b16, see prefill.hip)
 __device__ __forceinline__ f16x8 lds16_at(uint32_t byte) {
@@ -141,6 +177,7 @@ struct Block {
     f16x8 q[D / 16];
     f16x8 p[4];  // fp16 weights, then (LO) what they leave of the fp32 ones: B operands
     f32x16 s;
+    f16x2 wmin;  // LO: the least of the lane's weights of the unit, as fp16
     float m, l, psum;
 };
 
@@ -154,6 +191,13 @@ __device__ __forceinline__ void copy16(u32x4 r, uint32_t lds, uint32_t voff) {
         "buffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds),
         "v"(voff), "s"(r), "n"(OFF)
         : "memory", "scc");
+}
+
+// the lesser of each half; one instruction (the builtin quiets NaNs of both first)
+__device__ __forceinline__ f16x2 min_pair(f16x2 a, f16x2 b) {
+    f16x2 r;
+    asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
 }
 
 // weight pairs w[0..7] (and w[8..15]) as the B operands of their PV steps
@@ -398,6 +442,8 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
         }
     };
     const float scale = a.scale_log2;
+    constexpr float up = LO ? kUp : 0.f;
+    constexpr float kLimit = LO ? kSumLimitLo : kSumLimit;
     // P of the unit with the running maximum as it is, and the lane's sum of it
     // (of the weights PV multiplies: the fp16 ones, or with LO the fp32 ones)
     auto weights = [&](Block<D>& x) __attribute__((always_inline)) {
@@ -412,15 +458,17 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                 w[8 + j] = f16x2{(f16)(w0 - (float)(f16)w0), (f16)(w1 - (float)(f16)w1)};
             if constexpr (LO) x.psum += w0 + w1;
             else x.psum = add_pair(x.psum, w[j]);
+            if constexpr (LO) x.wmin = j == 0 ? w[0] : min_pair(x.wmin, w[j]);
         });
         operands<LO>(x.p, w);
     };
     // scores of unit u past the diagonal of block y, whose diagonal unit is d <= u
     auto mask = [&](Block<D>& y, uint32_t u, uint32_t d) __attribute__((always_inline)) {
-        const uint32_t top = u > d ? 0u : n + 1u;  // keys of the unit below it are visible
+        // keys of the unit up to n are visible; of the lane's, those below top
+        const int top = u > d ? 0 : (int)n + 1 - 4 * (int)hh;
         each<16>([&](auto e_tag) __attribute__((always_inline)) {
-            constexpr uint32_t e = decltype(e_tag)::value;
-            y.s[e] = 8u * (e >> 2) + 4u * hh + (e & 3u) >= top ? -INFINITY : y.s[e];
+            constexpr int e = decltype(e_tag)::value;
+            y.s[e] = 8 * (e >> 2) + (e & 3) >= top ? -INFINITY : y.s[e];
         });
     };
     auto unit_max = [&](const Block<D>& x) __attribute__((always_inline)) {
@@ -430,42 +478,131 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
         });
         return mx;
     };
+    // LO: whether a weight of the lane's unit is below kSmall
+    auto small = [&](const Block<D>& x) __attribute__((always_inline)) {
+        if constexpr (!LO) return false;
+        else {
+            // weights are not negative: as integers in their order
+            const u16x2 less = __builtin_bit_cast(u16x2, x.wmin) - kSmallBits;
+            return (__builtin_bit_cast(uint32_t, less) & 0x80008000u) != 0;
+        }
+    };
+    // ... and the least exponent of the unit's visible keys
+    auto unit_min = [&](const Block<D>& x) __attribute__((always_inline)) {
+        float mn = INFINITY;
+        each<16>([&](auto e_tag) __attribute__((always_inline)) {
+            constexpr int e = decltype(e_tag)::value;
+            mn = fminf(mn, x.s[e] == -INFINITY ? INFINITY : x.s[e]);
+        });
+        return __builtin_fmaf(mn, scale, -x.m);
+    };
+    // In accumulation registers the asm on O neither waits for MFMAs before it nor
+    // keeps those after it away: 32 wait states on both sides do
+    auto apart = [&](Block<D>& x) __attribute__((always_inline)) {
+        if constexpr (kAsm)
+            asm volatile("s_nop 15\n\ts_nop 15"
+                         : "+a"(x.o[0]), "+a"(x.o[1]), "+a"(x.o[2]), "+a"(x.o[3]));
+    };
+    // O times f
+    auto scale_o = [&](Block<D>& x, float f) __attribute__((always_inline)) {
+        apart(x);
+        each<4 * ND>([&](auto i_tag) __attribute__((always_inline)) {
+            constexpr int dt = decltype(i_tag)::value / 4, e = decltype(i_tag)::value % 4 * 4;
+            float v[4] = {x.o[dt][e], x.o[dt][e + 1], x.o[dt][e + 2], x.o[dt][e + 3]};
+            if constexpr (kAsm) {
+                scale_acc4(v[0], v[1], v[2], v[3], f);
+            } else {
+                v[0] *= f;
+                v[1] *= f;
+                v[2] *= f;
+                v[3] *= f;
+            }
+            x.o[dt][e] = v[0];
+            x.o[dt][e + 1] = v[1];
+            x.o[dt][e + 2] = v[2];
+            x.o[dt][e + 3] = v[3];
+        });
+        apart(x);
+    };
+    // What both halves leave of the weights of x's unit below kSmall, through a
+    // product of its own.  Weights from kSmall on leave nothing here, so that a
+    // row does not depend on the others.  The unit's V operands are at hand.
+    auto pv_rest = [&](Block<D>& x) __attribute__((always_inline)) {
+        f16x8 p[2];
+        // read back from the operands' registers; else they stay in others as well
+        each<4>([&](auto k_tag) __attribute__((always_inline)) {
+            f16x8& own = x.p[decltype(k_tag)::value];
+            asm volatile("" : "+v"(own));
+        });
+        each<8>([&](auto j_tag) __attribute__((always_inline)) {
+            constexpr int j = decltype(j_tag)::value, k = j / 4, i = j % 4 * 2;
+            f16x2 left;
+            each<2>([&](auto h_tag) __attribute__((always_inline)) {
+                constexpr int h = decltype(h_tag)::value;
+                const float w = fast_exp2(__builtin_fmaf(x.s[2 * j + h], scale, -x.m));
+                const f16 hi = x.p[k][i + h];
+                const float l = (w - (float)hi) - (float)x.p[2 + k][i + h];
+                left[h] = (f16)(hi < (f16)kSmall ? l * kUpRest : 0.f);
+            });
+            asm volatile("" : "+v"(left));  // one pair at a time: registers are short
+            p[k][i] = left[0];
+            p[k][i + 1] = left[1];
+        });
+        apart(x);
+        each<ND>([&](auto dt_tag) __attribute__((always_inline)) {
+            constexpr int dt = decltype(dt_tag)::value;
+            f32x16 t = mfma32(vf[0][dt], p[0], f32x16{});
+            t = mfma32(vf[1][dt], p[1], t);
+            if constexpr (kAsm) asm volatile("s_nop 15\n\ts_nop 15" : "+v"(t));
+            each<4>([&](auto i_tag) __attribute__((always_inline)) {
+                constexpr int e = 4 * decltype(i_tag)::value;
+                float v[4] = {x.o[dt][e], x.o[dt][e + 1], x.o[dt][e + 2], x.o[dt][e + 3]};
+                if constexpr (kAsm) {
+                    add_acc4(v[0], v[1], v[2], v[3], f32x4{t[e], t[e + 1], t[e + 2], t[e + 3]},
+                             1.f / kUpRest);
+                } else {
+                    v[0] = __builtin_fmaf(t[e], 1.f / kUpRest, v[0]);
+                    v[1] = __builtin_fmaf(t[e + 1], 1.f / kUpRest, v[1]);
+                    v[2] = __builtin_fmaf(t[e + 2], 1.f / kUpRest, v[2]);
+                    v[3] = __builtin_fmaf(t[e + 3], 1.f / kUpRest, v[3]);
+                }
+                x.o[dt][e] = v[0];
+                x.o[dt][e + 1] = v[1];
+                x.o[dt][e + 2] = v[2];
+                x.o[dt][e + 3] = v[3];
+            });
+        });
+        apart(x);
+    };
     // Between two phases.  x's weights of its unit are complete: raise the
     // maximum of the queries whose weights passed the limit (the two lanes of a
     // query together), rescale O and l and redo the unit.  y's scores of unit u
     // are complete: mask them past the diagonal, y's diagonal unit being d.  One
-    // test and one branch for both, rarely taken.
-    auto settle = [&](Block<D>& x, Block<D>& y, uint32_t u, uint32_t d)
-                      __attribute__((always_inline)) {
-        const uint64_t over_lanes = __builtin_amdgcn_ballot_w64(!(x.psum < kSumLimit));
-        if (__builtin_expect((over_lanes | (u >= d ? ~0ull : 0ull)) != 0, 0)) {
-            if (over_lanes) {
+    // test and one branch for both, rarely taken.  inside: x's unit is before its
+    // diagonal; lanes: those whose weights ask for it; get_v: the V operands of x's
+    // unit into vf.
+    auto settle = [&](Block<D>& x, bool inside, Block<D>& y, uint32_t u, uint32_t d,
+                      uint64_t lanes, auto&& get_v) __attribute__((always_inline)) {
+        if (__builtin_expect((lanes | (u >= d ? ~0ull : 0ull)) != 0, 0)) {
+            const bool over = !(x.psum < kLimit);
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(over) != 0, 0)) {
                 const float mx = unit_max(x);
-                const bool over = !(x.psum < kSumLimit);
                 const bool raise = max_xor<32>(over ? 1.f : 0.f) != 0.f;
-                const float m_unit = max_xor<32>(mx) * scale;
+                const float m_unit = max_xor<32>(mx) * scale - up;
                 const float mn = raise ? fmaxf(x.m, m_unit) : x.m;
                 const float al = fast_exp2(x.m - mn);
                 x.m = mn;
                 weights(x);
                 x.l *= al;
-                each<4 * ND>([&](auto i_tag) __attribute__((always_inline)) {
-                    constexpr int dt = decltype(i_tag)::value / 4, e = decltype(i_tag)::value % 4 * 4;
-                    float v[4] = {x.o[dt][e], x.o[dt][e + 1], x.o[dt][e + 2], x.o[dt][e + 3]};
-                    if constexpr (kAsm) {
-                        scale_acc4(v[0], v[1], v[2], v[3], al);
-                    } else {
-                        v[0] *= al;
-                        v[1] *= al;
-                        v[2] *= al;
-                        v[3] *= al;
-                    }
-                    x.o[dt][e] = v[0];
-                    x.o[dt][e + 1] = v[1];
-                    x.o[dt][e + 2] = v[2];
-                    x.o[dt][e + 3] = v[3];
-                });
-                if constexpr (kAsm) asm volatile("s_nop 7");
+                scale_o(x, al);
+            }
+            if constexpr (LO) {
+                // keys past the diagonal have weight 0, which is not small
+                const bool low = small(x) && (inside || unit_min(x) < -10.f);
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(low) != 0, 0)) {
+                    get_v();
+                    pv_rest(x);
+                }
             }
             if (u >= d) mask(y, u, d);
         }
@@ -473,10 +610,10 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
     };
     // before a block's first weights: the maximum of its first unit
     auto first_max = [&](Block<D>& x) __attribute__((always_inline)) {
-        x.m = fmaxf(kNoMax, max_xor<32>(unit_max(x)) * scale);
+        x.m = fmaxf(kNoMax, max_xor<32>(unit_max(x)) * scale - up);
     };
-    // B operand of PV step ks: the weights, then (ks 2, 3) what they leave
-    // PV MFMA f of block y: dim tile f % ND, step f / ND
+    // PV MFMA f of block y: dim tile f % ND, step f / ND (LO: the weights, then in steps
+    // 2 and 3 what they leave)
     auto pv = [&](Block<D>& y, auto f_tag) __attribute__((always_inline)) {
         constexpr int ks = decltype(f_tag)::value / ND, dt = decltype(f_tag)::value % ND;
         y.o[dt] = mfma32(vf[ks & 1][dt], y.p[ks], y.o[dt]);
@@ -495,7 +632,8 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
         const float mneg = -x.m;
         float psum[2] = {0.f, 0.f};
         float sh[16], ex[16];
-        f16x2 w[16];
+        f16x2 w[16], wmin;
+        uint64_t lanes = 0;
         [&]<int... SL>(std::integer_sequence<int, SL...>) {
             ([&] {
                 constexpr int sl = SL;
@@ -521,14 +659,23 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                         constexpr int e = 2 * J;
                         constexpr int f = J * (NS - 3) / 8;
                         if constexpr (sl == f + 2) {
-                            w[J] = f16x2{(f16)ex[e], (f16)ex[e + 1]};
+                            // LO: in asm, or the compiler converts again for the
+                            // operands (s_nop: v_exp_f32's result may be read one
+                            // instruction after it, which the compiler sees to for
+                            // instructions of its own only)
+                            if constexpr (LO)
+                                asm("s_nop 0\n\tv_cvt_pk_f16_f32 %0, %1, %2"
+                                    : "=v"(w[J])
+                                    : "v"(ex[e]), "v"(ex[e + 1]));
+                            else w[J] = f16x2{(f16)ex[e], (f16)ex[e + 1]};
                             if constexpr (LO) psum[J & 1] += ex[e] + ex[e + 1];
                             else psum[J & 1] = add_pair(psum[J & 1], w[J]);
                             asm volatile("" ::"v"(w[J]), "v"(psum[J & 1]));
                             if constexpr (LO) {
+                                wmin = J == 0 ? w[0] : min_pair(wmin, w[J]);
                                 w[8 + J] = f16x2{(f16)(ex[e] - (float)w[J][0]),
                                                  (f16)(ex[e + 1] - (float)w[J][1])};
-                                asm volatile("" ::"v"(w[8 + J]));
+                                asm volatile("" : "+v"(w[8 + J]) : "v"(wmin));
                             }
                         }
                         if constexpr (sl == f + 1) {
@@ -543,11 +690,18 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                         }
                     }(), ...);
                 }(std::make_integer_sequence<int, 8>{});
+                // every weight is there: which lanes have something for settle
+                if constexpr (sl == NS - 2) {
+                    x.psum = psum[0] + psum[1];
+                    if constexpr (LO) x.wmin = wmin;
+                    lanes = __builtin_amdgcn_ballot_w64(!(x.psum < kLimit)) |
+                            __builtin_amdgcn_ballot_w64(small(x));
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }(), ...);
         }(std::make_integer_sequence<int, NS>{});
         operands<LO>(x.p, w);
-        x.psum = psum[0] + psum[1];
+        return lanes;
     };
 
     using rK = std::integral_constant<int, 1>;
@@ -623,7 +777,8 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
         for (uint32_t i = 0; i < units; ++i) {
             if constexpr (KS == 4) next_k(ku);
             else next_stage(ku, lds0 + part * 2u * kUnitB);
-            phase(A, B, rK{}, ku, [&](auto sl_tag) __attribute__((always_inline)) {
+            uint64_t lanes =
+                phase(A, B, rK{}, ku, [&](auto sl_tag) __attribute__((always_inline)) {
                 constexpr int sl = decltype(sl_tag)::value;
                 if constexpr (KS == 4) {
                     // K of unit i has been read: its LDS takes unit i + 3's.  K of
@@ -644,10 +799,17 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                     if constexpr (sl == NK - 1) meet();
                 }
             });
-            settle(A, B, unit_of(i), dB);
+            settle(A, unit_of(i) < dA, B, unit_of(i), dB, lanes,
+                   [&]() __attribute__((always_inline)) {
+                // phase 1 is done with the V operands of unit i - 1
+                if constexpr (KS == 4) landed(std::integral_constant<int, rows64::kLeftV * NI>{});
+                each<2 * ND>([&](auto f) __attribute__((always_inline)) {
+                    load_v(vu, decltype(f)::value);
+                });
+            });
             if constexpr (KS == 4)  // V of unit i; K i + 3 may be in flight
                 landed(std::integral_constant<int, rows64::kLeftV * NI>{});
-            phase(B, A, rV{}, vu, [&](auto sl_tag) __attribute__((always_inline)) {
+            lanes = phase(B, A, rV{}, vu, [&](auto sl_tag) __attribute__((always_inline)) {
                 constexpr int sl = decltype(sl_tag)::value;
                 constexpr int c = sl - ND;  // the slots without operand reads
                 if constexpr (KS == 4) {
@@ -675,7 +837,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                     }
                 }
             });
-            settle(B, A, i + 1 < units ? unit_of(i + 1) : 0u, dA);
+            settle(B, unit_of(i) < dB, A, i + 1 < units ? unit_of(i + 1) : 0u, dA, lanes, []() {});
             if constexpr (KS == 4) next_v(vu);
             else vu = ku + kUnitB;
         }

@@ -117,3 +117,42 @@ def test_rows64_prefix_invariance(attn, gpu):
     for n in (705, 766, 960):
         part = run(attn, gpu, q[:n], k[:n], v[:n], 16, 4, 128, qs, ks)
         assert np.array_equal(part.view(np.uint16), whole[:n].view(np.uint16)), n
+
+
+def sink_inputs(N, Hq, Hkv, D, nats, sinks, seed):
+    """Keys `sinks` score about `nats` above the others and carry V = 0; V is large
+    enough that what the other keys leave is a normal fp16 value."""
+    rng = np.random.default_rng(seed)
+    u = rng.choice([-1.0, 1.0], (Hkv, D))
+    q = 2.0 * np.repeat(u, Hq // Hkv, 0)[None] + 0.2 * rng.standard_normal((N, Hq, D))
+    k = 0.3 * rng.standard_normal((N, Hkv, D))
+    v = 4096.0 * (1.0 + 0.3 * rng.standard_normal((N, Hkv, D)))
+    k[sinks] = nats / (2.0 * np.sqrt(D)) * u
+    v[sinks] = 0.0
+    return [x.reshape(N, -1).astype(np.float16) for x in (q, k, v)]
+
+
+# one sink in the first unit of 32 keys and in a later one, one in every unit;
+# both numbers of key parts
+@pytest.mark.parametrize("Hq,Hkv,D,N", [(4, 4, 128, 300), (8, 2, 64, 300), (32, 16, 128, 1100),
+                                        (16, 8, 64, 4161)])
+@pytest.mark.parametrize("sinks", [[0], [100], list(range(3, 300, 29))])
+@pytest.mark.parametrize("nats", [6, 12, 16, 20])
+def test_rows64_small_weights_beside_sinks(attn, gpu, Hq, Hkv, D, N, sinks, nats):
+    """Weights far below the largest keep their bits: no further from 64 bits than
+    attention_generic's fp32 weights (whose own error is the fp16 rounding of the
+    output; 2 % for another order of the sums)."""
+    q, k, v = sink_inputs(N, Hq, Hkv, D, nats, sinks, 13 + nats)
+    print(f"[case] rows64 sinks Hq={Hq} D={D} N={N} nats={nats} at={sinks[:2]}", flush=True)
+    args = (q, k, v, Hq, Hkv, D, Hq * D, Hkv * D)
+    rows = np.arange(1, N, 1 if N <= 300 else 23)
+    _, e32 = oracle.attention(q.view(np.uint16).ravel(), k.view(np.uint16).ravel(),
+                              v.view(np.uint16).ravel(), N, Hq, Hkv, D, Hq * D, Hkv * D, N,
+                              causal=True, rows=rows)
+    exact = e32.reshape(len(rows), -1).astype(np.float64)
+    got, ref = (run_(attn, gpu, *args)[rows].astype(np.float64) for run_ in (run, run_generic))
+    for name, part in (("all", slice(None)), ("first", rows < 128), ("last", rows >= N - 128)):
+        err = [np.linalg.norm(x[part] - exact[part]) / np.linalg.norm(exact[part])
+               for x in (got, ref)]
+        print(f"  {name}: {err[0]:.3e} against {err[1]:.3e}", flush=True)
+        assert err[0] <= 1.02 * err[1] + 1e-6, (name, err)
