@@ -445,10 +445,12 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
     constexpr float up = LO ? kUp : 0.f;
     constexpr float kLimit = LO ? kSumLimitLo : kSumLimit;
     // P of the unit with the running maximum as it is, and the lane's sum of it
-    // (of the weights PV multiplies: the fp16 ones, or with LO the fp32 ones)
+    // (of the weights PV multiplies: the fp16 ones, or with LO the fp32 ones),
+    // added in the order of `phase`: a row whose weights are only computed again
+    // because others' are keeps its bits
     auto weights = [&](Block<D>& x) __attribute__((always_inline)) {
         f16x2 w[16];
-        x.psum = 0.f;
+        float psum[2] = {0.f, 0.f};
         each<8>([&](auto j_tag) __attribute__((always_inline)) {
             constexpr int j = decltype(j_tag)::value;
             const float w0 = fast_exp2(__builtin_fmaf(x.s[2 * j], scale, -x.m));
@@ -456,11 +458,12 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
             w[j] = f16x2{(f16)w0, (f16)w1};
             if constexpr (LO)
                 w[8 + j] = f16x2{(f16)(w0 - (float)(f16)w0), (f16)(w1 - (float)(f16)w1)};
-            if constexpr (LO) x.psum += w0 + w1;
-            else x.psum = add_pair(x.psum, w[j]);
+            if constexpr (LO) psum[j & 1] += w0 + w1;
+            else psum[j & 1] = add_pair(psum[j & 1], w[j]);
             if constexpr (LO) x.wmin = j == 0 ? w[0] : min_pair(x.wmin, w[j]);
         });
         operands<LO>(x.p, w);
+        x.psum = psum[0] + psum[1];
     };
     // scores of unit u past the diagonal of block y, whose diagonal unit is d <= u
     auto mask = [&](Block<D>& y, uint32_t u, uint32_t d) __attribute__((always_inline)) {

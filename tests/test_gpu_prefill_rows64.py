@@ -119,6 +119,23 @@ def test_rows64_prefix_invariance(attn, gpu):
         assert np.array_equal(part.view(np.uint16), whole[:n].view(np.uint16)), n
 
 
+# the model's layout, and both numbers of key parts of the others
+@pytest.mark.parametrize("Hq,Hkv,D,N", [(16, 4, 128, 1000), (16, 16, 128, 300), (16, 4, 64, 300),
+                                        (32, 16, 128, 1100), (16, 8, 64, 4161)])
+def test_rows64_row_independence(attn, gpu, Hq, Hkv, D, N):
+    """A row's output does not depend on the other queries of its tile, bit for
+    bit, where their growing scores raise their maxima again and again."""
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, 0, 11)
+    others = np.arange(N) % 32 >= 16
+    sharp = q.copy()
+    sharp[others] *= np.float16(24)
+    print(f"[case] rows64 row independence Hq={Hq} Hkv={Hkv} D={D} N={N}", flush=True)
+    a = run(attn, gpu, q, k, v, Hq, Hkv, D, qs, ks)
+    b = run(attn, gpu, sharp, k, v, Hq, Hkv, D, qs, ks)
+    assert np.array_equal(a[~others].view(np.uint16), b[~others].view(np.uint16))
+    assert not np.array_equal(a[others], b[others])
+
+
 def sink_inputs(N, Hq, Hkv, D, nats, sinks, seed):
     """Keys `sinks` score about `nats` above the others and carry V = 0; V is large
     enough that what the other keys leave is a normal fp16 value."""
