@@ -864,7 +864,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float v = o[4 * i4 + e] * inv;
-                if constexpr (LO) bad = __builtin_fmaf(v, 0.f, bad);
+                bad = __builtin_fmaf(v, 0.f, bad);
                 w[e] = (f16)v;
             }
             *reinterpret_cast<f16x4*>(orow + 8 * i4) = w;
@@ -926,17 +926,15 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
             }
             store(blk, dt0 + d, o, inv);
         }
-        if constexpr (LO) {
-            // Rows with a value that is not finite are done again key by key: an
-            // MFMA multiplies the masked keys of a tile (weight 0) too, so an
-            // infinity or NaN in V reaches rows before it, and the two halves of
-            // a weight turn an infinity into a NaN.
-            uint64_t rows = __builtin_amdgcn_ballot_w64(bad != 0.f);
-            rows = (rows | rows >> 32) & 0xffffffffull;
-            for (; rows != 0; rows &= rows - 1)
-                plain_row(a, q0 + 32u * blk + (uint32_t)__builtin_ctzll(rows), head, g,
-                          32u * dt0, 32u * (uint32_t)kDt);
-        }
+        // Rows with a value that is not finite are done again key by key: an MFMA
+        // multiplies the masked keys of a tile (weight 0) too, so an infinity or NaN
+        // in V reaches rows before it, and the two halves of a weight (LO) turn an
+        // infinity into a NaN.
+        uint64_t rows = __builtin_amdgcn_ballot_w64(bad != 0.f);
+        rows = (rows | rows >> 32) & 0xffffffffull;
+        for (; rows != 0; rows &= rows - 1)
+            plain_row(a, q0 + 32u * blk + (uint32_t)__builtin_ctzll(rows), head, g,
+                      32u * dt0, 32u * (uint32_t)kDt);
     }
 }
 

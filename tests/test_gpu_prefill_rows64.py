@@ -136,6 +136,27 @@ def test_rows64_row_independence(attn, gpu, Hq, Hkv, D, N):
     assert not np.array_equal(a[others], b[others])
 
 
+@pytest.mark.parametrize("N", [705, 800, 1024])
+def test_rows64_model_layout_infinities_and_nans(attn, gpu, N):
+    """The model's layout: an infinity or NaN in V reaches exactly the rows that
+    see its key, not the earlier rows of the tile."""
+    Hq, Hkv, D = 16, 4, 128
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, 0, 6)
+    v[N - 30, 3] = np.inf
+    v[N - 20, D + 7] = np.nan
+    v[N - 10, 2 * D + 5] = -np.inf
+    v[500, 3 * D + 9] = np.inf
+    print(f"[case] rows64 model layout inf/nan N={N}", flush=True)
+    args = (q, k, v, Hq, Hkv, D, qs, ks)
+    got, ref = run(attn, gpu, *args), run_generic(attn, gpu, *args)
+    assert np.isfinite(ref[:500]).all() and not np.isfinite(ref[N - 1]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fine = np.isfinite(ref)
+    assert_close(np.where(fine, got, 0).astype(np.float16).reshape(-1).view(np.uint16),
+                 np.where(fine, ref, 0).astype(np.float32).reshape(-1), 2e-3, 1e-2, f"N={N}")
+
+
 def sink_inputs(N, Hq, Hkv, D, nats, sinks, seed):
     """Keys `sinks` score about `nats` above the others and carry V = 0; V is large
     enough that what the other keys leave is a normal fp16 value."""
