@@ -382,10 +382,10 @@ int attn_prefill_plan(const void* q, const void* k, const void* v, const void* o
  * workgroup per head and 32-query tile, its keys split over the waves and
  * combined through LDS, as 8 waves of 32 keys up to 32 tokens, 4 waves of
  * 64-key tiles up to 256 and 4 waves each streaming every 4th 32-key unit
- * above (query tiles of 64 tokens instead of 32 from 11/16 of a workgroup per
- * CU to two, 705 tokens for 16 heads); 1 = never, also no key halves; 2 = 4 waves of 64-key tiles (up to
- * 256 tokens); 3 = 8 waves of 32 keys (up to 256 tokens); 4 = the
- * streaming form at any length), "prefill_key_halves" (0 = automatic: from
+ * above (from 11/16 of a workgroup per CU to two, 705 tokens for 16 heads, a kernel of
+ * 64-query tiles with the same split); 1 = never, also no key halves; 2 = 4 waves of
+ * 64-key tiles (up to 256 tokens); 3 = 8 waves of 32 keys (up to 256 tokens); 4 = the
+ * streaming form of 32-query tiles at any length), "prefill_key_halves" (0 = automatic: from
  * 1025 to 4096 tokens, unless "prefill_waves" or "prefill_split_keys" is
  * set, 8-wave workgroups of 32 queries x 4 heads whose two 4-wave groups
  * take the even and the odd key tiles and combine through LDS; 1 = never;

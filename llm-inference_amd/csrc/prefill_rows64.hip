@@ -957,12 +957,12 @@ int rows64_parts(const PrefillArgs& a, bool mfma, int device) {
     const uint64_t wgs = (uint64_t)((a.seq_len + kRows - 1) / kRows) * a.num_heads;
     if (mfma) {
         // Part of the streaming split-keys form's range (the same units, split
-        // over the waves the same way), also when that form is asked for; the
-        // other forms of prefill.hip keep theirs, the key-halves tile from 1025
-        // tokens (where this kernel is ahead by 5-13 % up to 2048).
-        const long form = get_option(kOptPrefillSplitKeys);
-        if (a.seq_len > 1024u || (form != 0 && form != 4) || get_option(kOptPrefillWaves) ||
-            get_option(kOptPrefillStageAll) || get_option(kOptPrefillKeyHalves) == 2)
+        // over the waves the same way), unless an option asks for a form of
+        // prefill.hip; the key-halves tile keeps its range from 1025 tokens (where
+        // this kernel is ahead by 5-13 % up to 2048).
+        if (a.seq_len > 1024u || get_option(kOptPrefillSplitKeys) ||
+            get_option(kOptPrefillWaves) || get_option(kOptPrefillStageAll) ||
+            get_option(kOptPrefillKeyHalves) == 2)
             return 0;
         // From 11/16 of a workgroup per CU to two: fewer leave the shorter chains
         // of prefill_skn's 32-query workgroups ahead, more (160 KiB of LDS: one
