@@ -76,9 +76,9 @@ struct QkvGemmArgs {
 bool qkv_gemm_mfma_ok(const QkvGemmArgs& a);
 // fused: only when qkv_gemm_mfma_ok (hipErrorInvalidValue otherwise)
 hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t stream);
-// qkv_short.hip: the tile for a short prompt, or -1 (qkv_gemm_mfma_ok is the
-// caller's to check)
-int qkv_short_tile(const QkvGemmArgs& a, int device);
+// qkv_short.hip: the tile for a short prompt and what its rounds cost (tenths of a
+// microsecond at K = 2048), or -1 (qkv_gemm_mfma_ok is the caller's to check)
+int qkv_short_tile(const QkvGemmArgs& a, int device, uint64_t& cost);
 hipError_t launch_qkv_gemm_short(const QkvGemmArgs& a, int tile, bool fused, hipStream_t stream);
 
 hipError_t launch_qkv_kernel(const QkvArgs& a, bool fused, hipStream_t stream);

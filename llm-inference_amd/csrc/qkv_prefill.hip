@@ -586,7 +586,7 @@ constexpr Tile kTiles[] = {
 // 33.7 / 47.4, 2600 - / 40.0 / 54.7 / 47.9, 4100 - / 68.6 / 59.3 / 54.6 / 68.5,
 // 5200 - / 75.8 / 68.1 / 64.0 / 73.6, 6400 - / 90.4 / 93.0 / 104.9 / 84.4, 8192
 // - / 110 / 99.9 / 107 / 92.1.
-int pick_tile(const QkvGemmArgs& a, int device) {
+int pick_tile(const QkvGemmArgs& a, int device, uint64_t& least) {
     const long forced = get_option(kOptQkvGemmTokensPerWave), wide = get_option(kOptQkvGemmWide);
     const auto wide_fits = [&](uint32_t features) {
         return a.N % features == 0 && a.K % kWBK == 0 && aligned16(a.y);
@@ -595,7 +595,6 @@ int pick_tile(const QkvGemmArgs& a, int device) {
     if (forced == 32 || forced == 64 || forced == 128) return forced == 32 ? 0 : forced == 64 ? 1 : 2;
     const uint64_t cus = (uint64_t)device_cu_count(device);
     int best = -1;
-    uint64_t least = 0;
     for (int i = 0; i < 5; ++i) {
         const Tile& t = kTiles[i];
         if (i >= 3 && (wide == 1 || !wide_fits(t.features))) continue;
@@ -632,9 +631,17 @@ hipError_t launch_qkv_gemm_kernel(const QkvGemmArgs& a, bool fused, hipStream_t 
     }
     int device = 0;
     if (hipError_t e = hipGetDevice(&device)) return e;
-    if (const int tile = qkv_short_tile(a, device); tile >= 0)
-        return launch_qkv_gemm_short(a, tile, fused, stream);
-    switch (pick_tile(a, device)) {
+    // A short prompt takes the tiles of qkv_short.hip while their rounds cost less:
+    // against the 64 x 128 tile, us, weights from HBM, 128 tokens, K = 2048: N = 3072
+    // 9.7 / 16.8, 6144 12.8 / 17.7; 256 tokens: 11.6 / 16.5 and 19.7 / 17.6; N =
+    // 9216, K = 3072: 64 tokens 19.5 / 28.0, 192 30.3 / 26.7; N = 18432, K = 6144: 64
+    // tokens 76.8 / 65.6, 128 100.7 / 99.3 (128 x 128: 75.6)
+    uint64_t cost = 0, short_cost = 0;
+    const int tile = pick_tile(a, device, cost);
+    const int short_tile = qkv_short_tile(a, device, short_cost);
+    if (short_tile >= 0 && short_cost < cost)
+        return launch_qkv_gemm_short(a, short_tile, fused, stream);
+    switch (tile) {
         case 0: return launch_mfma<1>(a, fused, stream);
         case 1: return launch_mfma<2>(a, fused, stream);
         case 2: return launch_mfma<4>(a, fused, stream);

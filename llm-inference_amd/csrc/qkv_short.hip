@@ -284,11 +284,13 @@ constexpr Tile kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {32, 16}, {16, 16}};
 }  // namespace
 
 // The tile with the least rounds of workgroups times rows of a tile, which is
-// what the copies of a CU take (-1: the tiles of qkv_prefill.hip).  At 64 tokens
-// 32 x 32 (192 workgroups of 64 rows) takes 8.4 us, 64 x 32 (96 of 96 rows) 9.9.
-// Up to 256 tokens: beyond, the tiles add k-values in one order whatever their
-// size.  Below K = 1024 a wave has two units or less, nothing for a ring.
-int qkv_short_tile(const QkvGemmArgs& a, int device) {
+// what the copies of a CU take (-1: the tiles of qkv_prefill.hip), and their cost
+// on the scale of qkv_prefill.hip's tiles: 8.1 us for a round of 128 rows at K =
+// 2048.  At 64 tokens 32 x 32 (192 workgroups of 64 rows) takes 8.4 us, 64 x 32 (96
+// of 96 rows) 9.9.  Up to 256 tokens: beyond, the tiles add k-values in one order
+// whatever their size.  Below K = 1024 a wave has two units or less, nothing for a
+// ring.
+int qkv_short_tile(const QkvGemmArgs& a, int device, uint64_t& cost) {
     if (a.M > 256u || a.K < 1024u || get_option(kOptQkvGemmTokensPerWave) ||
         get_option(kOptQkvGemmWide) == 2)
         return -1;
@@ -304,6 +306,7 @@ int qkv_short_tile(const QkvGemmArgs& a, int device) {
             least = rows;
         }
     }
+    cost = least * 81u / 128u;
     return best;
 }
 

@@ -50,3 +50,20 @@ def test_short_prompt_fused_64_dim_heads_bitexact(attn, gpu, M, start_pos, rotat
     fy, fc, ty, tc, _ = fused_case(attn, gpu, M, start_pos, rotate, Hq, Hkv, 64, 1024)
     assert np.array_equal(fy, ty), "y"
     assert np.array_equal(fc, tc), "cache"
+
+
+# where the rounds of the short tiles cost more than those of the tiles for longer
+# prompts (256 CUs), the latter run: their bits are those of any of them
+@pytest.mark.parametrize("M,N,short", [(128, 6144, True), (192, 6144, False), (256, 6144, False),
+                                       (64, 9216, True), (192, 9216, False), (256, 12288, False),
+                                       (32, 18432, True), (64, 18432, False), (128, 18432, False)])
+def test_short_tiles_only_where_cheaper(attn, gpu, M, N, short):
+    print(f"[case] short or long M={M} N={N}", flush=True)
+    x, w = rand_inputs(M, N, 1024, M + N)
+    y = run_gemm(attn, gpu, x, w)
+    try:
+        attn.set_option("qkv_gemm_tokens_per_wave", 64)
+        ref = run_gemm(attn, gpu, x, w)
+    finally:
+        attn.set_option("qkv_gemm_tokens_per_wave", 0)
+    assert np.array_equal(y, ref) != short
