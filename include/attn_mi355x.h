@@ -254,7 +254,10 @@ int attn_decode_out_proj(const attn_f16_t* q, const attn_f16_t* k_cache, const a
  * accumulation, fp16 out, all row-major and packed.  seq_len == 0 or
  * total_qkv_dim == 0 is a no-op; hidden_size == 0 writes zeros (x, W may then
  * be null).  fp16 MFMA when hidden_size % 64 == 0 and x, W are 16-byte
- * aligned; any other shape runs a plain fp32-accumulating kernel. */
+ * aligned; any other shape runs a plain fp32-accumulating kernel.  The order in
+ * which an output's products are added depends on the shape, up to 256 tokens on
+ * seq_len too: a token's values agree between calls of different seq_len within the
+ * rounding of fp32 sums, bit for bit from 257 tokens on only. */
 int attn_qkv_gemm(const attn_f16_t* x, attn_f16_t* y, const attn_f16_t* w, size_t seq_len,
                   size_t hidden_size, size_t total_qkv_dim, hipStream_t stream);
 

@@ -579,8 +579,9 @@ struct Tile {
 constexpr Tile kTiles[] = {
     {64, 128, 130}, {128, 128, 165}, {256, 128, 250}, {256, 256, 460}, {256, 384, 660}};
 
-// The tile whose rounds cost least.  All tiles add a feature's k-values in the
-// same order, so the choice never shows in the results.  N = 3072, us for 64 x
+// The tile whose rounds cost least.  These tiles all add a feature's k-values in the
+// same order, so the choice among them never shows in the results; the short
+// prompt's tiles (qkv_short.hip) add in orders of their own.  N = 3072, us for 64 x
 // 128 / 128 x 128 / 256 x 128 / 256 x 256 / 256 x 384 tiles: 512 tokens 13.1 /
 // 15.9 / 24.4, 999 21.4 / 18.6 / 25.6, 1280 24.2 / 20.0 / 25.7, 2500 - / 39.5 /
 // 33.7 / 47.4, 2600 - / 40.0 / 54.7 / 47.9, 4100 - / 68.6 / 59.3 / 54.6 / 68.5,

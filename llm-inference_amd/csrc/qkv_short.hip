@@ -18,7 +18,9 @@
 //  * the waves split K: wave w takes the 64-value units w, w + W, ... with a
 //    ring of copies (buffer_load ... lds) of its own, computes the whole tile
 //    for them, and the W fp32 tiles are added through LDS at the end, in wave
-//    order.  No barrier stands between the first copy and the sum, so the waves
+//    order (so the last bit of a token's projection depends on W, that is on the
+//    tile and with it on how many tokens share the call; one order for 4 and 8
+//    waves costs the 64 x 64 tile 3 %).  No barrier stands between the first copy and the sum, so the waves
 //    do not wait for each other's copies.
 //  * LDS rows are the 128 bytes of a unit (whole cache lines: with 64-byte
 //    units the two halves of a line are fetched twice, 15.3 us at 254 tokens),
@@ -287,8 +289,8 @@ constexpr Tile kTiles[] = {{64, 64}, {64, 32}, {32, 32}, {32, 16}, {16, 16}};
 // what the copies of a CU take (-1: the tiles of qkv_prefill.hip), and their cost
 // on the scale of qkv_prefill.hip's tiles: 8.1 us for a round of 128 rows at K =
 // 2048.  At 64 tokens 32 x 32 (192 workgroups of 64 rows) takes 8.4 us, 64 x 32 (96
-// of 96 rows) 9.9.  Up to 256 tokens: beyond, the tiles add k-values in one order
-// whatever their size.  Below K = 1024 a wave has two units or less, nothing for a
+// of 96 rows) 9.9.  Up to 256 tokens: beyond, the tiles of qkv_prefill.hip alone
+// give every length one order of the k-values.  Below K = 1024 a wave has two units or less, nothing for a
 // ring.
 int qkv_short_tile(const QkvGemmArgs& a, int device, uint64_t& cost) {
     if (a.M > 256u || a.K < 1024u || get_option(kOptQkvGemmTokensPerWave) ||
