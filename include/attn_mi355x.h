@@ -83,7 +83,8 @@ int attn_prefill(const attn_f16_t* q, const attn_f16_t* k, const attn_f16_t* v,
  * kernel follows and exits at once, so that an updater can move the pair to
  * a longer context); other shapes enqueue one generic kernel and both
  * handles receive it, except head_dim 64 without node handles (16-byte
- * aligned tensors, a workspace): a split and a merge kernel of their own, in
+ * aligned tensors, a workspace, at least 64, 104 or 192 keys by the query heads per
+ * KV head: up to 2, up to 7, 8 and more): a split and a merge kernel of their own, in
  * fp32 like the generic kernel, which attn_update_decode_node and
  * attn_update_merge_node patch together through either node (never past the
  * states that the capturing call's kv_len asks for).

@@ -687,7 +687,7 @@ int attn_decode(const attn_f16_t* q, const attn_f16_t* k_cache, const attn_f16_t
         d.group = (uint32_t)(num_heads / num_kv_heads);
         d.capacity = (uint32_t)((kv_len + ATTN_KV_CHUNK - 1) / ATTN_KV_CHUNK);
         d.scale_log2 = scale_log2_for(head_dim);
-        if (plan_decode_d64(d, device)) {
+        if (decode_d64_pays(d.kv_len, d.group) && plan_decode_d64(d, device)) {
             e = launch_decode_d64_split(d, stream);
             if (e != hipSuccess) return (int)e;
             remember_launch<DecodeD64Args>(stream);

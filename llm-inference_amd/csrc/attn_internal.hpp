@@ -265,6 +265,8 @@ struct DecodeD64Args {
 };
 // fills nsplit and chunk; false: attention_generic takes the call
 bool plan_decode_d64(DecodeD64Args& a, int device);
+// false: a context so short that attention_generic is faster
+bool decode_d64_pays(uint32_t kv_len, uint32_t group);
 const void* decode_d64_split_symbol(const DecodeD64Args& a);
 const void* decode_d64_merge_symbol();
 bool is_decode_d64_split(const void* fn);

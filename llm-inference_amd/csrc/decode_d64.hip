@@ -243,6 +243,17 @@ bool plan_decode_d64(DecodeD64Args& a, int device) {
     return true;
 }
 
+// Whether two kernels take less than attention_generic's one.  That takes 3 us and
+// 0.035 per key; these 4.7-5.2 us up to 256 keys with 1 or 2 heads per workgroup,
+// 6.6-6.8 with 4, 9.4-9.6 with 8 (a merge that waits for the split, and the split's
+// code, which grows with the heads).  us at 16/4 heads, two kernels / one: 32 keys
+// 6.7 / 4.1, 100 6.65 / 6.57, 128 6.8 / 7.6; 8/8: 32 4.9 / 4.1, 64 4.9 / 5.3; 16/2:
+// 100 9.5 / 6.5, 200 9.5 / 10.0.
+bool decode_d64_pays(uint32_t kv_len, uint32_t group) {
+    const uint32_t hpw = heads_per_workgroup(group);
+    return kv_len >= (hpw <= 2 ? 64u : hpw == 4 ? 104u : 192u);
+}
+
 const void* decode_d64_split_symbol(const DecodeD64Args& a) { return split_symbol(a.group); }
 const void* decode_d64_merge_symbol() { return reinterpret_cast<const void*>(&decode_d64_merge); }
 bool is_decode_d64_split(const void* fn) {

@@ -88,6 +88,63 @@ def test_decode_d64_large_scores_and_nan(attn, gpu):
     assert_as_generic(np.where(where, 0, got), np.where(where, 0, ref), np.nan_to_num(v[:L]))
 
 
+def captured(attn, d, out, ws, L, Hq, Hkv, stride):
+    """One captured call of L keys: graph, executable graph, its last node, its
+    number of kernels."""
+    import ctypes
+    stream = torch.cuda.Stream()
+    sp = stream.cuda_stream
+    torch.cuda.synchronize()
+    hipgraph.begin_capture(sp)
+    attn.decode(*d, out, *ws, 1, L, L - 1, Hq, Hkv, D, 0, stride, stream=sp)
+    node = hipgraph.last_captured_node(sp)
+    graph, exe = hipgraph.end_capture(sp)
+    n = ctypes.c_size_t()
+    assert hipgraph._hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    return stream, graph, exe, node, n.value
+
+
+@pytest.mark.parametrize("Hq,Hkv,least", [(8, 8, 64), (4, 2, 64), (6, 2, 104), (16, 4, 104),
+                                          (16, 2, 192), (12, 1, 192)])
+def test_decode_d64_from_where_it_is_faster(attn, gpu, Hq, Hkv, least):
+    """The shortest context of the two kernels; below it the one generic kernel runs,
+    bit for bit."""
+    (q, k, v), d = inputs(least, Hq, Hkv, Hkv * D, 6, gpu)
+    ws, _ = workspace(attn, Hq, least, gpu)
+    out = torch.zeros(Hq * D, dtype=torch.float16, device=gpu)
+    for L, kernels in ((1, 1), (least - 1, 1), (least, 2)):
+        print(f"[case] decode d64 route Hq={Hq} Hkv={Hkv} L={L}", flush=True)
+        stream, graph, exe, _, n = captured(attn, d, out, ws, L, Hq, Hkv, Hkv * D)
+        hipgraph.destroy(graph, exe)
+        assert n == kernels, (L, n)
+        if kernels == 1:
+            got, ref = (f(attn, d, L, Hq, Hkv, Hkv * D, gpu) for f in (decode, generic))
+            assert np.array_equal(got.view(np.uint16), ref.view(np.uint16))
+
+
+# contexts below those, through a captured pair moved to them
+@pytest.mark.parametrize("Hq,Hkv,pad", [(16, 4, 0), (8, 8, 0), (4, 2, 8), (6, 2, 0), (16, 2, 0),
+                                        (12, 1, 24)])
+def test_decode_d64_short_contexts_of_a_patched_pair(attn, gpu, Hq, Hkv, pad):
+    stride, L0 = Hkv * D + pad, 1000
+    (q, k, v), d = inputs(L0, Hq, Hkv, stride, 7, gpu)
+    ws, _ = workspace(attn, Hq, L0, gpu)
+    out = torch.zeros(Hq * D, dtype=torch.float16, device=gpu)
+    stream, graph, exe, node, n = captured(attn, d, out, ws, L0, Hq, Hkv, stride)
+    assert n == 2
+    try:
+        for L in (1, 7, 12, 31, 64, 65, 127, L0):
+            print(f"[case] decode d64 patched Hq={Hq} Hkv={Hkv} L={L}", flush=True)
+            assert attn.lib().attn_update_decode_node(exe, node, L) == 0
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            hipgraph.launch(exe, stream.cuda_stream)
+            hipgraph.synchronize(stream.cuda_stream)
+            assert_as_generic(out.cpu().numpy(), generic(attn, d, L, Hq, Hkv, stride, gpu), v[:L])
+    finally:
+        hipgraph.destroy(graph, exe)
+
+
 @pytest.mark.parametrize("updater", ["decode", "merge", "split"])
 def test_decode_d64_captured_and_patched(attn, gpu, updater):
     """A captured call replays as the eager one; a node of it moves to other
