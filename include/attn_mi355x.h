@@ -360,9 +360,10 @@ int attn_decode_plan(size_t kv_len, size_t num_heads, size_t num_kv_heads, size_
                      const void* v_cache, uint32_t out[5]);
 
 /* Prefill path chosen for a shape: 1 = the MFMA tiles of four query heads per KV
- * head and head_dim 128, 0 = any other layout (head_dim 64 and 128 with 16-byte
- * aligned rows run the 64-rows-per-wave MFMA kernel from 64 tokens, everything
- * else the generic kernel). */
+ * head and head_dim 128, 0 = any other layout (with 16-byte aligned rows head_dim 64
+ * runs the 64-rows-per-wave MFMA kernel from 64 tokens, head_dim 128 from 64, 74 or
+ * 104 by the query heads, 20 and more, 10 and more, fewer; everything else the
+ * generic kernel). */
 int attn_prefill_plan(const void* q, const void* k, const void* v, const void* out,
                       size_t num_heads, size_t num_kv_heads, size_t head_dim, size_t q_stride,
                       size_t kv_stride);

@@ -972,9 +972,14 @@ int rows64_parts(const PrefillArgs& a, bool mfma, int device) {
         // 14.2, 1000 (512) 23 / 34; 8 heads 1000 (128) 14.1 / 12.7.
         return 16u * wgs > 11u * cus && wgs <= 2u * cus ? 4 : 0;
     }
-    // the other layouts ran attention_generic: ahead below 64 tokens (32: 5.5
-    // against 6.8 us at 16/16 heads of 128; 64: 7.6 against 7.4)
-    if (a.seq_len < 64) return 0;
+    // The other layouts ran attention_generic.  64-dim heads: level or ahead from 64
+    // tokens (1/1 heads 5.4 us against 5.3, 16/4 5.55 / 6.1).  128-dim heads take
+    // 7.4-7.6 us up to 100 tokens, attention_generic's grow with the heads: 64 tokens
+    // 1 head 6.2, 8 6.4, 16 7.2, 20 8.2; 80: 1 6.7, 8 7.1, 10 7.8; 104: 1 7.5, 4 7.8, 8 8.5
+    const uint32_t least = a.head_dim == 64 || a.num_heads >= 20 ? 64u
+                           : a.num_heads >= 10                   ? 74u
+                                                                 : 104u;
+    if (a.seq_len < least) return 0;
     // Four parts until the workgroups are two rounds of what the CUs hold (one
     // workgroup of 128-dim heads per CU, two of 64-dim heads), then two parts
     // and shared copies where pairs of heads share a KV head: 16/8 heads of 128
