@@ -20,6 +20,22 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
+#define LDS_AS __attribute__((address_space(3)))
+
+inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// s_waitcnt immediate that waits until at most n vector-memory operations are
+// outstanding (vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt not waited on)
+constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 0xF) | ((n >> 4) << 14); }
+static_assert(vmcnt_imm(0) == 0x0F70 && vmcnt_imm(16) == 0x4F70 && vmcnt_imm(63) == 0xCF7F);
+
+__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
 // 16-byte global load/store of eight fp16 values (pointer must be 16B aligned).
 __device__ __forceinline__ f16x8 ld16(const f16* p) {
     return *reinterpret_cast<const f16x8*>(p);

@@ -203,8 +203,6 @@ __global__ __launch_bounds__(256) void decode_d64_merge(DecodeD64Args a) {
     }
 }
 
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-
 uint32_t heads_per_workgroup(uint32_t group) {
     return group >= 8 ? 8u : group > 2 ? 4u : group;
 }

@@ -697,8 +697,6 @@ __global__ __launch_bounds__(64 * kMergeWaves) void flash_decode_merge(DecodeArg
 template <bool ROPE>
 __global__ __launch_bounds__(64 * kMergeWaves) void flash_decode_merge_idle(DecodeArgs) {}
 
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-
 }  // namespace
 
 int decode_hpw(int path) { return path == 1 ? 4 : path == 2 ? 2 : path == 3 ? 1 : 0; }

@@ -76,11 +76,6 @@ constexpr int kKDma = kBN * kKChunks / 64;    // 1 KiB DMA instructions per K ti
 constexpr int kVDma = kBN * kVChunks / 64;    // ... per V tile (16)
 constexpr int kMaxDma = kKDma > kVDma ? kKDma : kVDma;
 
-// s_waitcnt immediate that waits until at most n vector-memory loads are
-// outstanding (vmcnt bits 3:0 and 15:14; expcnt and lgkmcnt not waited on)
-constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 0xF) | ((n >> 4) << 14); }
-static_assert(vmcnt_imm(0) == 0x0F70 && vmcnt_imm(16) == 0x4F70 && vmcnt_imm(63) == 0xCF7F);
-
 // LDS chunk position pos of K row r holds the row's 16-byte chunk pos ^ (r % 16)
 __device__ __forceinline__ uint32_t k_src_chunk(uint32_t r, uint32_t pos) {
     return pos ^ (r & 15u);
@@ -97,15 +92,10 @@ __device__ __forceinline__ uint32_t v_src_chunk(uint32_t r, uint32_t pos) {
     return pos ^ (4u * (r & 3u));
 }
 
-#define LDS_AS __attribute__((address_space(3)))
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f16x8 lds16(const f16* p) {
     return *reinterpret_cast<const f16x8*>(p);
-}
-
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
 // Four fp16 of one LDS column: lane i of each 16-lane group receives element
@@ -1077,8 +1067,6 @@ __global__ __launch_bounds__(64 * kSknWaves, 1) void prefill_skn(PrefillArgs a) 
         }
     }
 }
-
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace
 

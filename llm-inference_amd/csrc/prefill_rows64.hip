@@ -79,13 +79,9 @@ constexpr float kUpRest = 0x1p36f;
 // weight 0 without a special case
 constexpr float kNoMax = -1.0e30f;
 
-#define LDS_AS __attribute__((address_space(3)))
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
 // The score MFMAs of one-wave-per-SIMD kernels, as inline assembly so that the
 // scores land in vector registers (the compiler puts every MFMA result of
 // such a kernel into accumulation registers and copies the scores back, 16
@@ -159,8 +155,6 @@ __device__ __forceinline__ void each(F&& f) {
         (f(std::integral_constant<int, I>{}), ...);
     }(std::make_integer_sequence<int, N>{});
 }
-constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 0xF) | ((n >> 4) << 14); }
-
 // blockIdx -> (head group, query tile): longest tiles first, head groups
 // pinned to XCDs when they divide the 8 of them
 __device__ __forceinline__ void map_block(uint32_t bid, uint32_t groups, uint32_t q_tiles,
@@ -937,8 +931,6 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
                       32u * dt0, 32u * (uint32_t)kDt);
     }
 }
-
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace
 

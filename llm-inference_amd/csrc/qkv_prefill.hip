@@ -45,14 +45,9 @@ constexpr int kBK = 64;      // k-values per stage
 constexpr int kRowH = kBK;   // halves per LDS row (128 B, no padding)
 constexpr int kThreads = 256;
 
-#define LDS_AS __attribute__((address_space(3)))
 
 __device__ __forceinline__ f16x8 lds16(const f16* p) {
     return *reinterpret_cast<const f16x8*>(p);
-}
-
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
 // blockIdx -> (token tile, feature tile).  Workgroups are dispatched
@@ -531,8 +526,6 @@ __global__ __launch_bounds__(256) void qkv_gemm_generic(QkvGemmArgs a) {
     for (uint32_t k = 0; k < a.K; ++k) acc += (float)xr[k] * (float)wr[k];
     a.y[(uint64_t)m * a.N + col] = (f16)acc;
 }
-
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 template <int WMT>
 hipError_t launch_mfma(const QkvGemmArgs& a, bool fused, hipStream_t stream) {

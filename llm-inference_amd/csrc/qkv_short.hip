@@ -42,12 +42,6 @@ namespace attn {
 
 namespace {
 
-__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
-
 // BM x BN tile, W waves, S units of each wave in its ring; P pairs of features
 // per thread in the epilogue
 template <int BM, int BN, int W, int S, int P, bool FUSED>

@@ -135,8 +135,6 @@ __global__ __launch_bounds__(256) void rope_store_kv_generic(RopeArgs a) {
     dst[i + half] = src[i + half];
 }
 
-inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
-
 }  // namespace
 
 bool rope_vector_ok(const RopeArgs& a) {
