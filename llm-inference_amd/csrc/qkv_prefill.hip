@@ -79,9 +79,13 @@ __device__ __forceinline__ void map_tile(uint32_t bid, uint32_t m_tiles, uint32_
 // One thread's columns of a fused tile of 128 features staged as [rows][64]
 // twice, features 0..63 and 64..127: 8 rotation pairs of a head, with the
 // destinations of the halves.  D = 128: the tile is one head, pairs (c, c + 64);
-// D = 64: two heads, threads 0-3 of a row the first, pairs (c, c + 32).
+// D = 64: two heads, threads 0-3 of a row the first, pairs (c, c + 32).  D is a
+// template parameter: read from the arguments it costs the 256 x 384 tiles 2 %
+// (fused, 16/4 heads of 128, 8192 tokens, 102.5 against 100.4 us).
+template <int D>
 struct FusedCols {
-    uint32_t head, half;        // half = D / 2
+    static constexpr uint32_t half = D / 2;
+    uint32_t head;
     uint32_t tcol;              // column of the first half, in the head and the table
     uint32_t col;               // ... in the tile
     uint32_t lo, hi;            // staged halves
@@ -90,28 +94,32 @@ struct FusedCols {
     uint64_t kv_dim;
     __device__ __forceinline__ FusedCols(const QkvGemmArgs& a, uint32_t tile, uint32_t j8,
                                          uint32_t rows) {
-        const bool d64 = a.head_dim == 64u;
-        const uint32_t second = d64 ? j8 >> 5 : 0u;
-        half = d64 ? 32u : 64u;
-        head = d64 ? 2u * tile + second : tile;
-        tcol = d64 ? j8 & 31u : j8;
+        const uint32_t second = D == 64 ? j8 >> 5 : 0u;
+        head = D == 64 ? 2u * tile + second : tile;
+        tcol = D == 64 ? j8 & 31u : j8;
         col = 64u * second + tcol;
         lo = second * rows * 64u + tcol;
-        hi = d64 ? lo + 32u : rows * 64u + j8;
+        hi = D == 64 ? lo + 32u : rows * 64u + j8;
         const uint32_t Hq = a.num_heads, Hkv = a.num_kv_heads;
         is_q = head < Hq;
         const bool is_k = !is_q && head < Hq + Hkv;
         rot = a.apply != 0 && (is_q || is_k);
-        kv_dim = (uint64_t)Hkv * a.head_dim;
+        kv_dim = (uint64_t)Hkv * D;
         cache = is_q ? nullptr
-                     : (is_k ? a.kc + (uint64_t)(head - Hq) * a.head_dim
-                             : a.vc + (uint64_t)(head - Hq - Hkv) * a.head_dim);
+                     : (is_k ? a.kc + (uint64_t)(head - Hq) * D
+                             : a.vc + (uint64_t)(head - Hq - Hkv) * D);
     }
+    // table(cs, sn): the row's entries, asked for where the head rotates
+    template <typename Table>
     __device__ __forceinline__ void store(const QkvGemmArgs& a, const f16* staged, uint32_t m,
-                                          uint32_t n0, f16x8 cs, f16x8 sn) const {
+                                          uint32_t n0, Table&& table) const {
         const f16x8 x0 = lds16(staged + lo), x1 = lds16(staged + hi);
         f16x8 r0 = x0, r1 = x1;
-        if (rot) rope_rotate8(x0, x1, cs, sn, r0, r1);
+        if (rot) {
+            f16x8 cs, sn;
+            table(cs, sn);
+            rope_rotate8(x0, x1, cs, sn, r0, r1);
+        }
         f16* yr = a.y + (uint64_t)m * a.N + n0 + col;
         if (is_q) {
             st16(yr, r0);
@@ -126,7 +134,8 @@ struct FusedCols {
     }
 };
 
-template <int WMT, bool FUSED>
+// D: head_dim of the fused kernel, 0 for the plain one
+template <int WMT, int D>
 __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     constexpr int BM = 64 * WMT;
     constexpr int kADma = BM * 8 / 64;        // 1 KiB DMA instructions per X stage
@@ -297,7 +306,7 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     __syncthreads();
     const uint32_t N = a.N;
     const uint32_t j8 = 8u * ((uint32_t)tid & 7u), rsub = (uint32_t)tid >> 3;
-    if (!FUSED) {
+    if constexpr (D == 0) {
 #pragma unroll
         for (int p = 0; p < BM / 32; ++p) {
             const uint32_t row = 32u * p + rsub, m = m0 + row;
@@ -316,28 +325,31 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
                 }
             }
         }
-        return;
-    }
-    // fused: the tile is head n_tile (D = 128) or heads 2 n_tile and 2 n_tile + 1
-    // (D = 64; the second may lie past N)
-    const FusedCols f(a, n_tile, j8, BM);
-    if (f.head >= a.num_heads + 2u * a.num_kv_heads) return;
-    // table rows of all passes first (rows past M read row M - 1, unused)
-    f16x8 cs[BM / 32], sn[BM / 32];
-    if (f.rot) {
+    } else {
+        // fused: the tile is head n_tile (D = 128) or heads 2 n_tile and 2 n_tile + 1
+        // (D = 64; the second may lie past N)
+        const FusedCols<D> f(a, n_tile, j8, BM);
+        if (D == 64 && f.head >= a.num_heads + 2u * a.num_kv_heads) return;
+        // table rows of all passes first (rows past M read row M - 1, unused)
+        f16x8 cs[BM / 32], sn[BM / 32];
+        if (f.rot) {
+#pragma unroll
+            for (int p = 0; p < BM / 32; ++p) {
+                const uint32_t m = min(m0 + 32u * p + rsub, a.M - 1u);
+                const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
+                cs[p] = ld16(a.cos_t + t);
+                sn[p] = ld16(a.sin_t + t);
+            }
+        }
 #pragma unroll
         for (int p = 0; p < BM / 32; ++p) {
-            const uint32_t m = min(m0 + 32u * p + rsub, a.M - 1u);
-            const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
-            cs[p] = ld16(a.cos_t + t);
-            sn[p] = ld16(a.sin_t + t);
+            const uint32_t row = 32u * p + rsub, m = m0 + row;
+            if (m >= a.M) break;
+            f.store(a, lds + row * 64u, m, n0, [&](f16x8& c0, f16x8& s0) {
+                c0 = cs[p];
+                s0 = sn[p];
+            });
         }
-    }
-#pragma unroll
-    for (int p = 0; p < BM / 32; ++p) {
-        const uint32_t row = 32u * p + rsub, m = m0 + row;
-        if (m >= a.M) break;
-        f.store(a, lds + row * 64u, m, n0, cs[p], sn[p]);
     }
 }
 
@@ -361,7 +373,7 @@ constexpr int kWADma = kWBM * 8 / 64;                  // 1 KiB DMA instructions
 constexpr int kWATs = kWADma / 8;                      // X instructions per wave (4)
 constexpr uint32_t kWStageA = kWBM * kWBK * 2;         // bytes of X per stage
 
-template <int NT, bool FUSED>
+template <int NT, int D>
 __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
     constexpr int kWBN = 128 * NT;
     constexpr int kWDmaPerWave = (kWADma + kWBN * 8 / 64) / 8;
@@ -486,7 +498,7 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
         }
         __syncthreads();
         const uint32_t hn0 = n0 + 128u * h;  // first feature of the round's head
-        if (!FUSED) {
+        if constexpr (D == 0) {
 #pragma unroll
             for (int p = 0; p < kWBM / 64; ++p) {
                 const uint32_t row = 64u * p + rsub, m = m0 + row;
@@ -495,21 +507,24 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
                 st16(yr + j8, lds16(lo + row * 64u + j8));
                 st16(yr + 64u + j8, lds16(hi + row * 64u + j8));
             }
-            continue;
-        }
-        // fused: the round's tile is head hn0 / 128 (D = 128) or two heads (D = 64)
-        const FusedCols f(a, hn0 / 128u, j8, kWBM);
+        } else {
+            // fused: the round's tile is head hn0 / 128 (D = 128) or two heads (D = 64)
+            const FusedCols<D> f(a, hn0 / 128u, j8, kWBM);
+            // addresses are made in each round: kept from round to round they take
+            // registers that the accumulators need (12 spilled; 16/4 heads of 128, 8192
+            // tokens 101.8 against 98.2 us)
+            uint32_t r0 = rsub;
+            asm volatile("" : "+v"(r0));
 #pragma unroll
-        for (int p = 0; p < kWBM / 64; ++p) {
-            const uint32_t row = 64u * p + rsub, m = m0 + row;
-            if (m >= a.M) break;
-            f16x8 cs{}, sn{};
-            if (f.rot) {
-                const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
-                cs = ld16(a.cos_t + t);
-                sn = ld16(a.sin_t + t);
+            for (int p = 0; p < kWBM / 64; ++p) {
+                const uint32_t row = 64u * p + r0, m = m0 + row;
+                if (m >= a.M) break;
+                f.store(a, lds + row * 64u, m, hn0, [&](f16x8& cs, f16x8& sn) {
+                    const uint64_t t = ((uint64_t)a.start_pos + m) * f.half + f.tcol;
+                    cs = ld16(a.cos_t + t);
+                    sn = ld16(a.sin_t + t);
+                });
             }
-            f.store(a, lds + row * 64u, m, hn0, cs, sn);
         }
     }
 }
@@ -537,12 +552,13 @@ hipError_t launch_mfma(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
     const uint64_t blocks = m_tiles * b.n_tiles;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
     b.m_tiles = (uint32_t)m_tiles;
-    if (fused)
-        hipLaunchKernelGGL((qkv_gemm_mfma<WMT, true>), dim3((uint32_t)blocks), dim3(kThreads), 0,
-                           stream, b);
+    const dim3 grid((uint32_t)blocks), block(kThreads);
+    if (!fused)
+        hipLaunchKernelGGL((qkv_gemm_mfma<WMT, 0>), grid, block, 0, stream, b);
+    else if (a.head_dim == 64u)
+        hipLaunchKernelGGL((qkv_gemm_mfma<WMT, 64>), grid, block, 0, stream, b);
     else
-        hipLaunchKernelGGL((qkv_gemm_mfma<WMT, false>), dim3((uint32_t)blocks), dim3(kThreads), 0,
-                           stream, b);
+        hipLaunchKernelGGL((qkv_gemm_mfma<WMT, 128>), grid, block, 0, stream, b);
     return hipGetLastError();
 }
 
@@ -554,12 +570,13 @@ hipError_t launch_wide(const QkvGemmArgs& a, bool fused, hipStream_t stream) {
     b.m_tiles = (a.M + kWBM - 1u) / kWBM;
     const uint64_t blocks = (uint64_t)b.m_tiles * b.n_tiles;
     if (blocks > 0x7fffffffull) return hipErrorInvalidValue;
-    if (fused)
-        hipLaunchKernelGGL((qkv_gemm_wide<NT, true>), dim3((uint32_t)blocks), dim3(kWThreads), 0,
-                           stream, b);
+    const dim3 grid((uint32_t)blocks), block(kWThreads);
+    if (!fused)
+        hipLaunchKernelGGL((qkv_gemm_wide<NT, 0>), grid, block, 0, stream, b);
+    else if (a.head_dim == 64u)
+        hipLaunchKernelGGL((qkv_gemm_wide<NT, 64>), grid, block, 0, stream, b);
     else
-        hipLaunchKernelGGL((qkv_gemm_wide<NT, false>), dim3((uint32_t)blocks), dim3(kWThreads), 0,
-                           stream, b);
+        hipLaunchKernelGGL((qkv_gemm_wide<NT, 128>), grid, block, 0, stream, b);
     return hipGetLastError();
 }
 
