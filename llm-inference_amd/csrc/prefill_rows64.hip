@@ -964,13 +964,20 @@ int rows64_parts(const PrefillArgs& a, bool mfma, int device) {
         // 14.2, 1000 (512) 23 / 34; 8 heads 1000 (128) 14.1 / 12.7.
         return 16u * wgs > 11u * cus && wgs <= 2u * cus ? 4 : 0;
     }
-    // The other layouts ran attention_generic.  64-dim heads: level or ahead from 64
-    // tokens (1/1 heads 5.4 us against 5.3, 16/4 5.55 / 6.1).  128-dim heads take
-    // 7.4-7.6 us up to 100 tokens, attention_generic's grow with the heads: 64 tokens
-    // 1 head 6.2, 8 6.4, 16 7.2, 20 8.2; 80: 1 6.7, 8 7.1, 10 7.8; 104: 1 7.5, 4 7.8, 8 8.5
-    const uint32_t least = a.head_dim == 64 || a.num_heads >= 20 ? 64u
-                           : a.num_heads >= 10                   ? 74u
-                                                                 : 104u;
+    // The other layouts ran attention_generic, whose time grows with the heads, up to
+    // ~140 tokens this kernel's does not.  us, attention_generic / this: 64-dim heads, 64
+    // tokens 1 head 5.56 / 5.64, 2 5.69 / 5.83, 16 6.50 / 5.90; 68 tokens 1 5.78 / 5.71.
+    // 128-dim heads: 64 tokens 20 heads 8.44 / 7.81; 74 12 7.59 / 7.83, 16 8.15 / 7.77;
+    // 80 10 8.04 / 7.81, 12 7.78 / 7.85; 88 12 8.39 / 7.87; 104 4 8.08 / 8.20, 8 8.88 /
+    // 8.19; 112 2 8.13 / 8.42, 4 8.61 / 8.42; 136 1 8.81 / 8.83, 2 9.03 / 8.82
+    const uint32_t h = a.num_heads;
+    const uint32_t least = a.head_dim == 64 ? (h >= 8 ? 64u : 66u)
+                           : h >= 20        ? 64u
+                           : h >= 16        ? 74u
+                           : h >= 10        ? 84u
+                           : h >= 8         ? 104u
+                           : h >= 4         ? 112u
+                                            : 136u;
     if (a.seq_len < least) return 0;
     // Four parts until the workgroups are two rounds of what the CUs hold (one
     // workgroup of 128-dim heads per CU, two of 64-dim heads), then two parts

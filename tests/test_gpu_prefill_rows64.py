@@ -58,8 +58,9 @@ def assert_as_generic(got, ref, v):
 
 # the shortest prompt of the kernel by the number of heads; one token less is
 # attention_generic's, bit for bit
-@pytest.mark.parametrize("Hq,Hkv,D,least", [(20, 10, 128, 64), (10, 5, 128, 74), (16, 16, 128, 74),
-                                            (9, 9, 128, 104), (1, 1, 128, 104), (1, 1, 64, 64)])
+@pytest.mark.parametrize("Hq,Hkv,D,least", [(20, 10, 128, 64), (16, 16, 128, 74), (10, 5, 128, 84),
+                                            (9, 9, 128, 104), (4, 4, 128, 112), (3, 3, 128, 136),
+                                            (1, 1, 128, 136), (8, 8, 64, 64), (2, 1, 64, 66)])
 def test_rows64_from_where_it_is_faster(attn, gpu, Hq, Hkv, D, least):
     q, k, v, qs, ks = inputs(least, Hq, Hkv, D, 0, 9)
     for N in (least - 1, least):
@@ -75,7 +76,7 @@ def test_rows64_from_where_it_is_faster(attn, gpu, Hq, Hkv, D, least):
 # block long; past two rounds of workgroups (1041 and 576 of them) two key parts
 @pytest.mark.parametrize("Hq,Hkv,D,N,pad", [
     (16, 16, 128, 64, 0), (16, 16, 128, 65, 0), (20, 20, 128, 64, 0), (20, 10, 128, 65, 0),
-    (16, 16, 128, 74, 0), (3, 3, 128, 104, 0), (16, 8, 128, 97, 8), (6, 2, 128, 130, 24),
+    (16, 16, 128, 74, 0), (3, 3, 128, 136, 0), (16, 8, 128, 97, 8), (6, 2, 128, 130, 24),
     (5, 5, 128, 300, 0), (16, 16, 128, 1000, 0), (32, 16, 128, 1100, 8),
     (16, 4, 64, 64, 0), (16, 4, 64, 95, 8), (8, 8, 64, 128, 0), (3, 1, 64, 129, 16),
     (16, 4, 64, 1025, 0), (16, 8, 64, 4161, 0)])
