@@ -952,7 +952,7 @@ int rows64_parts(const PrefillArgs& a, bool mfma, int device) {
         // over the waves the same way), unless an option asks for a form of
         // prefill.hip; the key-halves tile keeps its range from 1025 tokens (where
         // this kernel is ahead by 5-13 % up to 2048).
-        if (a.seq_len > 1024u || get_option(kOptPrefillSplitKeys) ||
+        if (a.seq_len <= 256u || a.seq_len > 1024u || get_option(kOptPrefillSplitKeys) ||
             get_option(kOptPrefillWaves) || get_option(kOptPrefillStageAll) ||
             get_option(kOptPrefillKeyHalves) == 2)
             return 0;
@@ -961,8 +961,15 @@ int rows64_parts(const PrefillArgs& a, bool mfma, int device) {
         // per CU at a time) a third round.  us against prefill_skn: 16 heads 600
         // tokens (160 workgroups) 11.6 against 11.1, 800 (208) 12.6 / 14.7, 999
         // (256) 14.4 / 17.8; 32 heads 350 (192) 10.5 / 10.7, 500 (256) 11.4 /
-        // 14.2, 1000 (512) 23 / 34; 8 heads 1000 (128) 14.1 / 12.7.
-        return 16u * wgs > 11u * cus && wgs <= 2u * cus ? 4 : 0;
+        // 14.2, 1000 (512) 23 / 34; 8 heads 1000 (128) 14.1 / 12.7.  A second
+        // round pays from 417 tokens, or where prefill_skn's workgroups pass 9/4
+        // per CU: 64 heads 280 (576 of those) 14.6 / 13.9, 289 (640) 14.7 / 15.6, 48
+        // heads 340 (528) 14.6 / 13.4, 40 heads 400 (520) 14.5 / 13.5, 448 (560) 14.8 /
+        // 16.2.  Up to 256 tokens prefill_d128's all-tiles form: 64 heads 150 tokens
+        // 9.1 / 7.6, 192 10.0 / 8.6, 128 heads 150 14.6 / 11.7.
+        const uint64_t wgs32 = (uint64_t)((a.seq_len + 31) / 32) * a.num_heads;
+        if (16u * wgs <= 11u * cus || wgs > 2u * cus) return 0;
+        return wgs <= cus || a.seq_len > 416u || 4u * wgs32 > 9u * cus ? 4 : 0;
     }
     // The other layouts ran attention_generic, whose time grows with the heads, up to
     // ~140 tokens this kernel's does not.  us, attention_generic / this: 64-dim heads, 64

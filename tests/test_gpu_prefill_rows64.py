@@ -174,6 +174,31 @@ def test_rows64_model_layout_infinities_and_nans(attn, gpu, N):
                  np.where(fine, ref, 0).astype(np.float32).reshape(-1), 2e-3, 1e-2, f"N={N}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,N,form", [
+    # the all-tiles form up to 256 tokens, the 32-query streaming form where its
+    # workgroups are few, else this kernel
+    (64, 16, 150, 2), (64, 16, 256, 2), (128, 32, 65, 2), (128, 32, 192, 2),
+    (64, 16, 257, 4), (64, 16, 288, 4), (48, 12, 340, 4), (40, 10, 416, 4),
+    (64, 16, 289, 0), (40, 10, 417, 0), (96, 24, 257, 0), (40, 10, 384, 0)])
+def test_rows64_grouped_layout_routes(attn, gpu, Hq, Hkv, N, form):
+    """Many heads of the grouped layout: the form that is fastest there (256 CUs)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are in workgroups per CU, the sizes for 256 CUs")
+    D = 128
+    q, k, v, qs, ks = inputs(N, Hq, Hkv, D, 0, 10)
+    print(f"[case] rows64 grouped route Hq={Hq} N={N}", flush=True)
+    args = (q, k, v, Hq, Hkv, D, qs, ks)
+    got = run(attn, gpu, *args).view(np.uint16)
+    try:
+        attn.set_option("prefill_split_keys", form or 4)
+        forced = run(attn, gpu, *args).view(np.uint16)
+    finally:
+        attn.set_option("prefill_split_keys", 0)
+    assert np.array_equal(got, forced) == (form != 0)
+    assert_close(got.reshape(-1), forced.astype(np.uint16).view(np.float16).astype(np.float32)
+                 .reshape(-1), 2e-3, 1e-2, f"{Hq}/{Hkv} N={N}")
+
+
 def sink_inputs(N, Hq, Hkv, D, nats, sinks, seed):
     """Keys `sinks` score about `nats` above the others and carry V = 0; V is large
     enough that what the other keys leave is a normal fp16 value."""
