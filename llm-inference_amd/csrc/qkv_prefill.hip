@@ -153,6 +153,9 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_gemm_mfma(QkvGemmArgs a) {
     // stages are the explicit vmcnt + barrier of each step
     __shared__ __attribute__((aligned(16))) f16 lds[kStages * kStage / 2];
 
+    // The epilogue's arguments before the loop: a scalar load still in flight there
+    // makes its waits for LDS reads wait for all of them
+    if constexpr (D != 0) asm volatile("" ::"s"(a.start_pos), "s"(a.apply), "s"(a.num_heads));
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -380,6 +383,9 @@ __global__ __launch_bounds__(kWThreads, 1) void qkv_gemm_wide(QkvGemmArgs a) {
     constexpr uint32_t kWStage = kWStageA + kWBN * kWBK * 2;  // bytes per stage
     __shared__ __attribute__((aligned(16))) f16 lds[2 * kWStage / 2];
 
+    // The epilogue's arguments before the loop: a scalar load still in flight there
+    // makes its waits for LDS reads wait for all of them
+    if constexpr (D != 0) asm volatile("" ::"s"(a.start_pos), "s"(a.apply), "s"(a.num_heads));
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
