@@ -244,9 +244,10 @@ __device__ __forceinline__ void plain_row(const PrefillArgs& a, uint32_t row, ui
             s[i] = j0 + 64u * (uint32_t)i + lane <= row ? fast_exp2(s[i] - mn) : 0.f;
             sum += s[i];
         }
-#pragma unroll
+#pragma unroll 1
         for (int i = 0; i < 4; ++i) {
             const uint32_t first = j0 + 64u * (uint32_t)i;
+            const float w = i < 2 ? (i == 0 ? s[0] : s[1]) : (i == 2 ? s[2] : s[3]);
             if (first > row) break;
             const uint32_t keys = row - first + 1u;
             for (uint32_t j1 = 0; j1 < min(64u, keys); j1 += 16u) {
@@ -265,7 +266,7 @@ __device__ __forceinline__ void plain_row(const PrefillArgs& a, uint32_t row, ui
                 for (uint32_t e = 0; e < 16u; ++e) {
                     if (j1 + e >= keys) break;
                     const float p = __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i]), (int)(j1 + e)));
+                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), (int)(j1 + e)));
                     part[0] += p * (float)x[e][0];
                     part[1] += p * (float)x[e][1];
                 }
@@ -958,6 +959,7 @@ __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1, D == 64 ? 2 : 1))) void pref
             if (rows != 0) {
                 const uint32_t key = q0 + lane;
                 bool fault = false;
+#pragma unroll 1
                 for (uint32_t c = 0; key < N && c < 4u * (uint32_t)kDt; ++c) {
                     const f16x8 x = ld16(a.v + (uint64_t)key * a.kv_stride + (uint64_t)g * D +
                                          32u * dt0 + 8u * c);
