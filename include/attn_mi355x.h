@@ -354,16 +354,18 @@ const char* attn_weights_error_string(int code);
  * kernel serving 4, 2, 1 KV heads per workgroup), out[1] = splits of the
  * context, out[2] = keys per split, out[3] = threads per workgroup, out[4] =
  * partial states per query head written to the workspace (at most
- * ceil(kv_len / ATTN_KV_CHUNK)). */
+ * ceil(kv_len / ATTN_KV_CHUNK)).  The split and merge kernels of head_dim 64 are
+ * not among these plans: such calls answer path 0. */
 int attn_decode_plan(size_t kv_len, size_t num_heads, size_t num_kv_heads, size_t head_dim,
                      size_t kv_stride, const void* q, const void* k_cache,
                      const void* v_cache, uint32_t out[5]);
 
 /* Prefill path chosen for a shape: 1 = the MFMA tiles of four query heads per KV
- * head and head_dim 128, 0 = any other layout (with 16-byte aligned rows head_dim 64
- * runs the 64-rows-per-wave MFMA kernel from 64 tokens, head_dim 128 from 64, 74 or
- * 104 by the query heads, 20 and more, 10 and more, fewer; everything else the
- * generic kernel). */
+ * head and head_dim 128 (a part of whose prompts up to 1024 tokens run as 64 rows
+ * per wave, see "prefill_split_keys"), 0 = any other layout (with 16-byte aligned
+ * rows the 64-rows-per-wave MFMA kernel: head_dim 64 from 64 tokens, 66 below 8 query
+ * heads; head_dim 128 from 64 tokens at 20 heads and more, 74 at 16, 84 at 10, 104 at 8,
+ * 112 at 4, 136 below; everything else the generic kernel). */
 int attn_prefill_plan(const void* q, const void* k, const void* v, const void* out,
                       size_t num_heads, size_t num_kv_heads, size_t head_dim, size_t q_stride,
                       size_t kv_stride);
@@ -387,8 +389,9 @@ int attn_prefill_plan(const void* q, const void* k, const void* v, const void* o
  * workgroup per head and 32-query tile, its keys split over the waves and
  * combined through LDS, as 8 waves of 32 keys up to 32 tokens, 4 waves of
  * 64-key tiles up to 256 and 4 waves each streaming every 4th 32-key unit
- * above (from 11/16 of a workgroup per CU to two, 705 tokens for 16 heads, a kernel of
- * 64-query tiles with the same split); 1 = never, also no key halves; 2 = 4 waves of
+ * above (where 64-query tiles make 11/16 of a workgroup per CU and more, up to two, 705
+ * tokens for 16 heads, and not a second round of a few: a kernel of 64-query tiles
+ * with the same split); 1 = never, also no key halves; 2 = 4 waves of
  * 64-key tiles (up to 256 tokens); 3 = 8 waves of 32 keys (up to 256 tokens); 4 = the
  * streaming form of 32-query tiles at any length), "prefill_key_halves" (0 = automatic: from
  * 1025 to 4096 tokens, unless "prefill_waves" or "prefill_split_keys" is

@@ -1,7 +1,9 @@
-// Generic grouped-query attention for shapes the MFMA paths do not cover
-// (prefill: head_dim other than 64 and 128, fewer than 64 tokens of the layouts
-// prefill_rows64.hip takes; decode: head_dim != 128; unaligned or odd strides, e.g. the reference's Flash-Decode
-// known-answer test with D = 32 and kv_stride = kv_dim + 17).
+// Generic grouped-query attention for shapes that no other kernel covers.  Prefill:
+// head_dim other than 64 and 128, and prompts too short for prefill_rows64.hip
+// (rows64_parts).  Decode: head_dim other than 64 and 128, and of 64-dim heads short
+// contexts and calls with node handles or without a workspace (decode_d64.hip).
+// Both: unaligned or odd strides, e.g. the reference's Flash-Decode known-answer
+// test with D = 32 and kv_stride = kv_dim + 17.
 //
 // One 256-thread workgroup per (query row, query head).  Keys are streamed in
 // tiles of 256: each thread scores one key (fp32 dot product), the tile maximum

@@ -864,8 +864,8 @@ constexpr int kSknWaves = 4;
 // (32.0 against 32.4 us) and slower from 1664 (37.0 against 34.6 us), where
 // the 4x K/V reads of one-head workgroups outweigh their parallelism; from
 // 1025 tokens the key-halves tile is faster (1152 tokens 23.6 against 26.8 us)
-// (from 11/16 of a 64-query workgroup per CU to two, prefill_rows64.hip takes
-// this form's place with 64-query tiles)
+// (where 64-query tiles make 11/16 to two workgroups per CU, prefill_rows64.hip
+// takes most of this form's place with them: rows64_parts)
 constexpr uint32_t kSknMaxTokens = 1024;
 constexpr int kSknUnitBytes = 2 * kSkUnit * kD * 2;       // K + V of 32 keys: 16 KiB
 constexpr int kSknDma = kSknUnitBytes / 1024;             // 16: 8 for K, then 8 for V

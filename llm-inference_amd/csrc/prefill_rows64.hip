@@ -49,7 +49,8 @@
 // against prefill_skn at 16/4 heads of 128: 800 tokens 12.6 (14.7), 999 14.4
 // (17.8), 32/8 heads 1000 tokens 23 (34).  A phase takes
 // ~600 cycles for 512 cycles of MFMAs; short prompts are bound by the ~4 us of
-// first copies, code fetch and state fold, long ones by the power the MFMAs draw.
+// first copies (all of them: the compiler's wait for Q leaves none in flight), code
+// fetch and state fold, long ones by the power the MFMAs draw.
 #include "attn_internal.hpp"
 #include "rows64_copies.hpp"
 
